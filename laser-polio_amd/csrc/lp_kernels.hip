@@ -946,7 +946,7 @@ __device__ int64_t block_scan_nodes(int N, Cnt cnt, Emit emit) {
       v[a] = n < N ? cnt(n) : 0;
     }
     const int64_t sum = v[0] + v[1] + v[2] + v[3];
-    const int64_t incl = wave_incl_scan_i64(sum, lane);
+    const int64_t incl = wave_incl_scan_i64(sum);
     if (lane == 63) s_w[w] = incl;
     __syncthreads();
     int64_t off = carry + incl - sum, tot = 0;
@@ -1660,7 +1660,7 @@ __global__ void __launch_bounds__(WG, 5) k_full(Dev d, int mask) {
     // the span's RI / SIA exposures -> next day's list: one atomic per wave
     int c = 0;
     for (int u = 0; u < span0.z; ++u) c += __popc(s_sv[u][tid]);
-    const int incl = (int)wave_incl_scan_i64(c, lane);
+    const int incl = (int)wave_incl_scan_i64(c);
     const int tot = __shfl(incl, 63, 64);
     if (tot) {
       int base = 0;
@@ -2474,7 +2474,7 @@ __device__ int64_t node_span_scan(int64_t* partials, int64_t* prefix, int s0, in
         int64_t* p = partials + (size_t)s * NPART + P_SW;
         v = ATOMIC_IO ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
       }
-      const int64_t incl = wave_incl_scan_i64(v, lane);
+      const int64_t incl = wave_incl_scan_i64(v);
       if (s < s1) {
         const int64_t ex = carry + incl - v;
         if (ATOMIC_IO) __hip_atomic_store(prefix + s, ex, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2532,7 +2532,7 @@ __global__ void __launch_bounds__(WG) k_node_reduce(Dev d, int mask, int recount
   if (list) {
     if (lane_spans) {
       if (tid < 64) {
-        const int64_t incl = wave_incl_scan_i64(psw, tid);
+        const int64_t incl = wave_incl_scan_i64(psw);
         if (s0 + tid < s1) d.span_prefix[s0 + tid] = incl - psw;
         span_lane(incl - psw);
         if (tid == 63) s_w = incl;
@@ -2587,7 +2587,7 @@ __global__ void __launch_bounds__(WG) k_node_reduce(Dev d, int mask, int recount
       if (tid == 0) d.W_round[n] = s_w;            // the prefix was written above
     } else if (lane_spans) {
       if (tid < 64) {
-        const int64_t incl = wave_incl_scan_i64(psw, tid);
+        const int64_t incl = wave_incl_scan_i64(psw);
         if (s0 + tid < s1) d.span_prefix[s0 + tid] = incl - psw;
         span_lane(incl - psw);
         const int64_t W = __shfl(incl, 63, 64);
@@ -3000,7 +3000,7 @@ __device__ int64_t resolve_in_tiles(const Dev& d, int64_t tile0, int ntiles, int
   const int64_t c0 = tile0 * (LP_TILE / LP_CHUNK);
   const int nc = ntiles * (LP_TILE / LP_CHUNK);
   const int64_t cw = lane < nc ? ld64<ATOMIC_IO>(d.chunk_sum + c0 + lane) : 0;
-  const int64_t cincl = wave_incl_scan_i64(cw, lane);
+  const int64_t cincl = wave_incl_scan_i64(cw);
   const uint64_t cb = __ballot(lane < nc && sp_base + cincl > T);
   if (cb == 0) return -1;
   const int Lc = __ffsll((unsigned long long)cb) - 1;
@@ -3021,7 +3021,7 @@ __device__ int64_t resolve_in_tiles(const Dev& d, int64_t tile0, int ntiles, int
     w[a] = s_like ? weight_q24(lane_of(rk, a)) : 0;
   }
   const int64_t lsum = w[0] + w[1] + w[2] + w[3];
-  const int64_t incl = wave_incl_scan_i64(lsum, lane);
+  const int64_t incl = wave_incl_scan_i64(lsum);
   int64_t cum = cp + (incl - lsum);
   int hit = -1;
   for (int a = 0; a < 4; ++a) { cum += w[a]; if (hit < 0 && cum > T) hit = a; }
@@ -3413,7 +3413,7 @@ __global__ void __launch_bounds__(WG) k_finish(Dev d) {
         const int64_t v = my_span ? __hip_atomic_load(d.partials + (size_t)(s0 + lane) * NPART + P_SW, __ATOMIC_RELAXED,
                                                       __HIP_MEMORY_SCOPE_AGENT)
                                   : 0;
-        const int64_t incl = wave_incl_scan_i64(v, lane);
+        const int64_t incl = wave_incl_scan_i64(v);
         W = __shfl(incl, 63, 64);
         if (my_span) spx = incl - v;
       } else {
