@@ -104,6 +104,7 @@ struct lp_ctx {
   int32_t tpw = 4;
   int32_t agent_grid = 1;
   int32_t ei_grid = 2048, sample_grid = 2048;     // launch shapes of the list pass and the sampler
+  bool finish_wide = false;                       // k_finish with 1024 threads a node (no more nodes than CUs)
   bool mix_wide = false;                          // k_mix_foi<4> (more nodes than resident waves)
   int32_t mix_tiles = 0;                           // mix_mode 1: 16-row tiles of the largest simulation
   std::vector<void*> allocs;
@@ -351,7 +352,10 @@ int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool ad
     const size_t off_lds = (N + 1 <= lp::LDS_OFF_MAX) ? (size_t)(N + 1) * sizeof(int64_t) : 0;
     if (!off_lds) hipLaunchKernelGGL(lp::k_plan, dim3(1), dim3(lp::WG), 0, s, d, 1);
     hipLaunchKernelGGL(lp::k_sample, dim3(c->sample_grid), dim3(lp::WG), off_lds, s, d);
-    hipLaunchKernelGGL(lp::k_finish, dim3(N), dim3(lp::WG), 0, s, d);
+    if (c->finish_wide)
+      hipLaunchKernelGGL((lp::k_finish<1024, 4>), dim3(N), dim3(1024), 0, s, d);
+    else
+      hipLaunchKernelGGL((lp::k_finish<512, 6>), dim3(N), dim3(512), 0, s, d);
   }
   hipLaunchKernelGGL(lp::k_day_end, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask, tx_adjust, advance ? 1 : 0);
   HIPCHK(c, hipGetLastError());
@@ -527,6 +531,9 @@ int lp_prepare(lp_ctx* c) {
     // k_mix_foi: the variant held to 4 waves per SIMD once its workgroups outnumber those
     // of the unrestricted variant resident at once
     const int mix_blocks = (int)grid_of(N, lp::WG / 64);
+    // k_finish: 1024 threads a node while every node's workgroup is resident at once (one a
+    // CU); above that 512 threads held to 6 waves per SIMD (three a CU)
+    c->finish_wide = N <= cus;
     c->mix_wide = mix_blocks > resident(reinterpret_cast<const void*>(lp::k_mix_foi<1>), 0, 1 << 30);
   }
   int4* spans_d; int32_t* nspan_d;
@@ -581,7 +588,6 @@ int lp_prepare(lp_ctx* c) {
   if ((rc = alloc(c, &d.birth_dbg, 2 * (size_t)N))) return rc;
   if ((rc = alloc(c, &d.size, N))) return rc;
   if ((rc = alloc(c, &d.take_all, N))) return rc;
-  if ((rc = alloc(c, &d.n_uniq, N))) return rc;
   if ((rc = alloc(c, &d.m_round, N))) return rc;
   if ((rc = alloc(c, &d.resv, N))) return rc;
   if ((rc = alloc(c, &d.W_round, N))) return rc;

@@ -128,7 +128,7 @@ struct Dev {
   int32_t* ri_lcnt;        // [2][nodes] their lengths
   float* p_dbg; float* expected_dbg; int64_t* total_dbg; float* beta_mixed;
   int64_t* birth_dbg;      // [nodes][2] integer part and fraction threshold of the last VD step's expected births
-  int32_t* size; int32_t* take_all; int32_t* n_uniq; int32_t* m_round; int64_t* W_round;
+  int32_t* size; int32_t* take_all; int32_t* m_round; int64_t* W_round;
   uint64_t* thr_strain; int32_t* newexp;
   int64_t* probe_off; int64_t* round_base; uint64_t* sel_list; int64_t* sel_count; int64_t sel_cap;
   uint32_t* sel_word;      // [sel_cap] round 1: a claimed agent's selection weight (all ones: recompute)
@@ -227,7 +227,7 @@ __device__ __forceinline__ DayBeginIn day_begin_load(const Dev& d, int n, int32_
 }
 __device__ __forceinline__ void day_begin_apply(const Dev& d, int n, int32_t t, const DayBeginIn& in) {
   for (int k = 0; k < LP_MAX_STRAINS; ++k) d.newexp[n * LP_MAX_STRAINS + k] = 0;
-  d.n_uniq[n] = 0; d.size[n] = 0; d.take_all[n] = 0; d.m_round[n] = 0;
+  d.size[n] = 0; d.take_all[n] = 0; d.m_round[n] = 0;
   d.births[n] = 0;
   d.nb_begin[n] = in.live_end;
   d.ei_cnt[(size_t)((t + 1) & 1) * d.n_nodes + n] = 0;
@@ -2986,111 +2986,218 @@ __device__ __forceinline__ int64_t ld64(const int64_t* p) {
   return ATOMIC_IO ? __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : *p;
 }
 
-// The agent hit by target T inside the span of `ntiles` tiles from tile `tile0`,
-// whose prefix (weight before it) is sp_base: the chunk by a wave scan of the span's
-// chunk weights, the agent by a wave scan of the chunk's agent weights (S agents,
-// state 0, weigh).  ATOMIC_IO: the weights and states are read with atomic loads
-// (other wavefronts change them during the kernel).  MARKED_AS_S: an agent claimed
-// earlier in the round (SEL_MARK) keeps its weight, so that every probe of a round
-// sees the weights of the round's start.  Returns the slot, or -1 if the weights were
-// inconsistent; *word (when given) receives the hit agent's state word as read here.
-template <bool ATOMIC_IO, bool MARKED_AS_S>
-__device__ int64_t resolve_in_tiles(const Dev& d, int64_t tile0, int ntiles, int64_t sp_base, int64_t T, int lane,
-                                    uint32_t* word = nullptr) {
-  const int64_t c0 = tile0 * (LP_TILE / LP_CHUNK);
-  const int nc = ntiles * (LP_TILE / LP_CHUNK);
-  const int64_t cw = lane < nc ? ld64<ATOMIC_IO>(d.chunk_sum + c0 + lane) : 0;
-  const int64_t cincl = wave_incl_scan_i64(cw);
-  const uint64_t cb = __ballot(lane < nc && sp_base + cincl > T);
-  if (cb == 0) return -1;
-  const int Lc = __ffsll((unsigned long long)cb) - 1;
-  const int64_t cp = sp_base + __shfl(cincl, Lc, 64) - __shfl(cw, Lc, 64);
-  const int64_t c = c0 + Lc;
-  const int64_t i0 = c * LP_CHUNK + (int64_t)lane * 4;
-  uint32_t st4;
-  if (ATOMIC_IO || MARKED_AS_S)
-    st4 = __hip_atomic_load(reinterpret_cast<const uint32_t*>(d.state) + (i0 >> 2), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else
-    st4 = reinterpret_cast<const uint32_t*>(d.state)[i0 >> 2];
-  const float4 rk = *reinterpret_cast<const float4*>(d.risk + i0);
-  int64_t w[4];
+// A wavefront resolves up to PROBE_ROWS probes of one node at once, one per row of 16
+// lanes: the chain of dependent steps of a probe (span, chunk weights, agents) is
+// latency, so four of them in flight cost about what one did.  With one probe per
+// wavefront k_sample took 34 us a day and k_finish 39 us on the 14-node year (4.5 M
+// agents), 72 and 119 us on 64 replicates; now 17 and 24, 51 and 65 us with k_finish's
+// workgroups as before, less with the larger ones below.
+constexpr int PROBE_ROWS = 4;
+
+// The state words of 16 agents from 16-byte aligned `st`.
+template <bool ATOMIC_IO>
+__device__ __forceinline__ void load_states16(const int8_t* st, uint32_t (&w)[4]) {
+  if (ATOMIC_IO) {
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const uint32_t b = (st4 >> (8 * a)) & 0xffu;
-    const bool s_like = b == 0 || (MARKED_AS_S && b == (uint32_t)(uint8_t)SEL_MARK);
-    w[a] = s_like ? weight_q24(lane_of(rk, a)) : 0;
+    for (int v = 0; v < 4; ++v)
+      w[v] = __hip_atomic_load(reinterpret_cast<const uint32_t*>(st) + v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    const uint4 x = *reinterpret_cast<const uint4*>(st);
+    w[0] = x.x; w[1] = x.y; w[2] = x.z; w[3] = x.w;
   }
-  const int64_t lsum = w[0] + w[1] + w[2] + w[3];
-  const int64_t incl = wave_incl_scan_i64(lsum);
-  int64_t cum = cp + (incl - lsum);
-  int hit = -1;
-  for (int a = 0; a < 4; ++a) { cum += w[a]; if (hit < 0 && cum > T) hit = a; }
-  const uint64_t hb = __ballot(hit >= 0);
-  if (hb == 0) return -1;
-  const int L = __ffsll((unsigned long long)hb) - 1;
-  const int ha = __shfl(hit, L, 64);
-  if (word) *word = __shfl(st4, L, 64);
-  return c * LP_CHUNK + (int64_t)L * 4 + ha;
 }
 
-// resolve_in_tiles over span s.
-template <bool ATOMIC_IO, bool MARKED_AS_S>
-__device__ __forceinline__ int64_t resolve_in_span(const Dev& d, int64_t s, int64_t sp_base, int64_t T, int lane,
-                                                   uint32_t* word = nullptr) {
-  const int4 span = d.spans[s];
-  return resolve_in_tiles<ATOMIC_IO, MARKED_AS_S>(d, span.y, span.z, sp_base, T, lane, word);
+// 0x80 in every byte of the state word that is 0 (or SEL_MARK), 0 in the others: per byte,
+// (b & 0x7f) + 0x7f reaches bit 7 unless the low bits are 0.
+template <bool MARKED_AS_S>
+__device__ __forceinline__ uint32_t s_like_bytes(uint32_t w) {
+  const uint32_t z = ~(((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u;
+  if (!MARKED_AS_S) return z;
+  const uint32_t y = w ^ 0x7f7f7f7fu;
+  static_assert(SEL_MARK == 0x7f, "SEL_MARK byte");
+  return z | (~(((y & 0x7f7f7f7fu) + 0x7f7f7f7fu) | y) & 0x80808080u);
 }
 
-
-// One wavefront per probe: target T in [0, W); the span with prefix <= T by a
-// 64-ary search over the node's span prefix, the chunk inside the span by a wave
-// scan of its chunk weights, the agent inside the chunk by a wave scan of the
-// agents' weights (ATOMIC_IO, MARKED_AS_S as for resolve_in_tiles).  Returns the
-// slot, or -1 if the weights were inconsistent.
+// The last stage of resolve_row when a risk reaches 256 (a weight of 2^32): the same sums
+// and search one agent at a time in 64 bits, from memory again.
 template <bool ATOMIC_IO, bool MARKED_AS_S>
-__device__ int64_t resolve_probe(const Dev& d, int node, int64_t T, const int64_t* prefix, int lane,
-                                 uint32_t* word = nullptr) {
-  int64_t lo = d.node_span_begin[node];
-  int64_t hi = d.node_span_begin[node + 1];   // search spans [lo, hi)
+__device__ __forceinline__ int64_t resolve_row_wide(const Dev& d, int64_t i0, bool on, int64_t cp, int64_t T,
+                                                    uint32_t& word) {
+  uint32_t st[4] = {~0u, ~0u, ~0u, ~0u};
+  if (on) load_states16<ATOMIC_IO>(d.state + i0, st);
+  auto weight = [&](int a) -> int64_t {
+    const uint32_t w = a < 4 ? st[0] : a < 8 ? st[1] : a < 12 ? st[2] : st[3];
+    return on && ((s_like_bytes<MARKED_AS_S>(w) >> (8 * (a & 3) + 7)) & 1u) ? weight_q24(d.risk[i0 + a]) : 0;
+  };
+  int64_t lsum = 0;
+#pragma unroll 1
+  for (int a = 0; a < 16; ++a) lsum += weight(a);
+  int64_t cum = cp + (row_incl_scan_i64(lsum) - lsum);
+  if (!on || cum > T || cum + lsum <= T) return -1;
+  int hit = 0;
+#pragma unroll 1
+  for (; hit < 15; ++hit) {
+    cum += weight(hit);
+    if (cum > T) break;
+  }
+  word = hit < 4 ? st[0] : hit < 8 ? st[1] : hit < 12 ? st[2] : st[3];
+  return i0 + hit;
+}
+
+// The probe of this lane's row: the agent hit by target T inside the span of `ntiles`
+// (at most 16) tiles from tile `tile0`, whose prefix (weight before it) is sp_base.  Lane
+// rl = lane % 16 of the row takes the four chunk weights of tile rl, a row scan gives the
+// chunk; then 16 agents of that chunk, and a row scan of their weights (S agents, state 0,
+// weigh) the agent.  Rows without a probe pass ntiles 0; every lane of the wave calls.
+// ATOMIC_IO: the weights and states are read with atomic loads (other wavefronts change
+// them during the kernel).  MARKED_AS_S: an agent claimed earlier in the round
+// (SEL_MARK) keeps its weight, so that every probe of a round sees the weights of the
+// round's start (a state word read before or after such a claim weighs the same, so it
+// needs no atomic load).  Returns the slot in the lane that holds the agent and -1 in
+// the others (in all of them if the weights were inconsistent); `word`: that lane's state
+// word of the agent as read here.
+template <bool ATOMIC_IO, bool MARKED_AS_S>
+__device__ __forceinline__ int64_t resolve_row(const Dev& d, int64_t tile0, int ntiles, int64_t sp_base, int64_t T,
+                                               int lane, uint32_t& word) {
+  const int rl = lane & 15, r0 = lane & 48;
+  int64_t cw[4] = {0, 0, 0, 0};
+  if (rl < ntiles) {
+    const int64_t* c = d.chunk_sum + (tile0 + rl) * (LP_TILE / LP_CHUNK);
+    if (ATOMIC_IO) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) cw[q] = ld64<true>(c + q);
+    } else {                                              // 32-byte aligned: a tile's four chunks
+      const longlong2 lo = reinterpret_cast<const longlong2*>(c)[0], hi = reinterpret_cast<const longlong2*>(c)[1];
+      cw[0] = lo.x; cw[1] = lo.y; cw[2] = hi.x; cw[3] = hi.y;
+    }
+  }
+  const int64_t ts = (cw[0] + cw[1]) + (cw[2] + cw[3]);
+  const int64_t tincl = row_incl_scan_i64(ts);
+  const uint32_t tb = (uint32_t)(__ballot(rl < ntiles && sp_base + tincl > T) >> r0) & 0xffffu;
+  const int Lt = tb ? __ffs((int)tb) - 1 : 0;            // the row's tile (none: no lane returns a slot)
+  // the chunk of the lane's own tile that T falls into, and the weight before it
+  int64_t cp = sp_base + tincl - ts;
+  int q = 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+    if (q == a && cp + cw[a] <= T) { cp += cw[a]; q = a + 1; }
+  q = __shfl(q, r0 + Lt, 64);
+  cp = __shfl(cp, r0 + Lt, 64);
+  const int64_t i0 = ((tile0 + Lt) * (LP_TILE / LP_CHUNK) + q) * LP_CHUNK + (int64_t)rl * 16;
+  uint32_t st[4] = {~0u, ~0u, ~0u, ~0u};
+  uint32_t x[16];                                        // the agents' weights (S agents, below 2^32)
+  bool wide = false;
+  {
+    float4 rk[4];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) rk[v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (tb) {
+      load_states16<ATOMIC_IO>(d.state + i0, st);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) rk[v] = *reinterpret_cast<const float4*>(d.risk + i0 + 4 * v);
+    }
+    float top = 0.0f;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const uint32_t m = s_like_bytes<MARKED_AS_S>(st[v]);
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        // weight_q24 (0 for negative values and NaN) in 32 bits
+        const float f = __builtin_rintf(__builtin_fmaxf(lane_of(rk[v], a), 0.0f) * 16777216.0f);
+        top = __builtin_fmaxf(top, f);
+        const uint32_t w = f < 4294967296.0f ? (uint32_t)f : 0u;
+        x[4 * v + a] = w & (uint32_t)((int32_t)(m << (24 - 8 * a)) >> 31);
+      }
+    }
+    wide = top >= 4294967296.0f;
+  }
+  if (__ballot(wide) != 0) return resolve_row_wide<ATOMIC_IO, MARKED_AS_S>(d, i0, tb != 0, cp, T, word);
+  int64_t g[4];
+#pragma unroll
+  for (int v = 0; v < 4; ++v) g[v] = ((int64_t)x[4 * v] + x[4 * v + 1]) + ((int64_t)x[4 * v + 2] + x[4 * v + 3]);
+  const int64_t lsum = (g[0] + g[1]) + (g[2] + g[3]);
+  int64_t rem = T - (cp + (row_incl_scan_i64(lsum) - lsum));
+  if (!tb || rem < 0 || rem >= lsum) return -1;          // not the row's lane
+  int hv = 0;
+#pragma unroll
+  for (int v = 0; v < 3; ++v)
+    if (hv == v && rem >= g[v]) { rem -= g[v]; hv = v + 1; }
+  uint32_t y[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) y[a] = hv == 0 ? x[a] : hv == 1 ? x[4 + a] : hv == 2 ? x[8 + a] : x[12 + a];
+  int ha = 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a)
+    if (ha == a && rem >= (int64_t)y[a]) { rem -= y[a]; ha = a + 1; }
+  word = hv == 0 ? st[0] : hv == 1 ? st[1] : hv == 2 ? st[2] : st[3];
+  return i0 + 4 * hv + ha;
+}
+
+// The span of a node with more than 64 spans that holds target T (the same in every
+// lane): the last one of [lo, hi) with prefix <= T, by a 64-ary search.
+template <bool ATOMIC_IO>
+__device__ int64_t search_span(const int64_t* prefix, int64_t lo, int64_t hi, int64_t T, int lane) {
   while (hi - lo > 1) {
     const int64_t range = hi - lo;
     const int64_t step = (range + 63) / 64;
     const int64_t c = lo + (int64_t)lane * step;
     const int64_t v = (c < hi) ? ld64<ATOMIC_IO>(prefix + c) : INT64_MAX;
     const uint64_t ok = __ballot(v <= T);        // monotone: lane 0 always true
-    const int L = 63 - __clzll(ok);
-    lo = lo + (int64_t)L * step;
+    lo += (int64_t)(63 - __clzll((unsigned long long)ok)) * step;
     const int64_t nhi = lo + step;
     hi = nhi < hi ? nhi : hi;
   }
-  const int64_t s = lo;
-  return resolve_in_span<ATOMIC_IO, MARKED_AS_S>(d, s, ld64<ATOMIC_IO>(prefix + s), T, lane, word);
+  return lo;
 }
 
-// Claim a hit: state byte 0 -> SEL_MARK with a word CAS; false if the agent was
-// already claimed (a duplicate probe) or is not susceptible.
-__device__ __forceinline__ bool claim(int8_t* state, int64_t slot) {
-  uint32_t* w = reinterpret_cast<uint32_t*>(state) + (slot >> 2);
-  const int sh = 8 * (int)(slot & 3);
-  uint32_t old = __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  while (true) {
-    if (((old >> sh) & 0xffu) != 0) return false;
-    const uint32_t nw = (old & ~(0xffu << sh)) | ((uint32_t)(uint8_t)SEL_MARK << sh);
-    const uint32_t prev = atomicCAS(w, old, nw);
-    if (prev == old) return true;
-    old = prev;
+// Where each row's probe continues: the span of the node that holds its target.  `np`
+// probes (rows 0 .. np - 1, targets T, the same across a row) of one node of `ns` spans
+// from span s0; up to 64 spans lane l holds span l's prefix (spx, INT64_MAX past the
+// last), first tile and tiles, above them `prefix` is searched.
+struct RowSpan {
+  int64_t tile0, base;
+  int ntiles;
+};
+template <bool ATOMIC_IO>
+__device__ __forceinline__ RowSpan row_spans(const Dev& d, int np, int64_t T, int ns, int s0, int64_t spx, int stile,
+                                             int sntile, const int64_t* prefix, int lane) {
+  RowSpan rs{0, 0, 0};
+  const int row = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < PROBE_ROWS; ++r) {
+    if (r >= np) break;
+    const int64_t Tr = readlane_i64(T, 16 * r);
+    int64_t base;
+    int tile, nt;
+    if (ns <= 64) {
+      const uint64_t ok = __ballot(spx <= Tr);            // monotone over the node's spans
+      const int L = ok ? 63 - __clzll((unsigned long long)ok) : 0;
+      base = readlane_i64(spx, L);
+      tile = __builtin_amdgcn_readlane(stile, L);
+      nt = ok ? __builtin_amdgcn_readlane(sntile, L) : 0;
+    } else {
+      const int64_t s = search_span<ATOMIC_IO>(prefix, s0, (int64_t)s0 + ns, Tr, lane);
+      base = ld64<ATOMIC_IO>(prefix + s);
+      const int4 span = d.spans[s];
+      tile = span.y;
+      nt = span.z;
+    }
+    if (row == r) { rs.tile0 = tile; rs.base = base; rs.ntiles = nt; }
   }
+  return rs;
 }
 
-// claim() starting from the state word `seen` (the word read when the agent was
-// resolved, its byte then S): the first compare-and-swap needs no load before it,
-// and a word changed since costs one more attempt with the value it returns.
-__device__ __forceinline__ bool claim_from(int8_t* state, int64_t slot, uint32_t seen) {
+// Claim a hit: state byte 0 -> `to` with a word CAS; false if the agent was already
+// claimed (a duplicate probe) or is not susceptible.  It starts from the state word
+// `seen` (read when the agent was resolved, its byte then S): the first
+// compare-and-swap needs no load before it, and a word changed since costs one more
+// attempt with the value it returns.
+__device__ __forceinline__ bool claim_from(int8_t* state, int64_t slot, uint32_t seen, int8_t to) {
   uint32_t* w = reinterpret_cast<uint32_t*>(state) + (slot >> 2);
   const int sh = 8 * (int)(slot & 3);
   uint32_t old = seen & ~(0xffu << sh);
   while (true) {
-    const uint32_t nw = old | ((uint32_t)(uint8_t)SEL_MARK << sh);
+    const uint32_t nw = old | ((uint32_t)(uint8_t)to << sh);
     const uint32_t prev = atomicCAS(w, old, nw);
     if (prev == old) return true;
     if (((prev >> sh) & 0xffu) != 0) return false;
@@ -3125,11 +3232,12 @@ __device__ __forceinline__ int expose_agent_thr(const Dev& d, const uint64_t* th
   return k;
 }
 
-constexpr uint64_t SEL_WON = 1ull << 63;   // round-1 entry whose probe claimed its agent
+constexpr uint64_t SEL_WON = 1ull << 63;   // round-1 entry whose probe claimed its agent,
+constexpr int SEL_STRAIN = 40;             // whose strain is in bits 40-41
 
 // Sampling round 1, grid-wide: one wavefront per probe resolves it to an agent, and
 // the first probe of each agent hit claims it (the round's distinct agents, counted
-// per node in n_uniq).  Every probe of the round must see the weights of the round's
+// by k_finish).  Every probe of the round must see the weights of the round's
 // start, so a claimed agent keeps its weight and reads as S (state SEL_MARK) until
 // k_finish makes it E and removes its weight; its strain, record byte and entry for
 // tomorrow's list are written here.  Probe j of node n owns position resv[n] + j of
@@ -3166,9 +3274,11 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
   } else {
     M = d.probe_off[N];
   }
-  const int64_t nw = (int64_t)gridDim.x * (WG / 64);
-  const int64_t first = (int64_t)blockIdx.x * (WG / 64);
-  if (first >= M) return;
+  // probe numbers fit 32 bits (M <= sel_cap), and each wave's are the same in all its lanes
+  const int Mp = __builtin_amdgcn_readfirstlane((int)M);
+  const int nw = (int)gridDim.x * (WG / 64);
+  if ((int)blockIdx.x * (WG / 64) >= Mp) return;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int64_t* off = lds ? s_off : d.probe_off;
   const int4 dy = today(d);
   const int32_t t = dy.x;
@@ -3179,59 +3289,63 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
   // node's seed, weight and span prefix (one span per lane, up to 64 spans) are
   // loaded once per node within a group of 64 probes, so a probe costs the
   // chunk-weight and the agent loads
-  const int64_t per = (M + nw - 1) / nw;
-  const int64_t p0 = (first + (threadIdx.x >> 6)) * per;
-  const int64_t p1 = p0 + per < M ? p0 + per : M;
-  // groups of up to 64 probes: resolved one at a time by the whole wave into the wave's
+  const int per = (Mp - 1) / nw + 1;
+  const int64_t first = (int64_t)((int)blockIdx.x * (WG / 64) + wave) * per;   // grids and M below 2^31
+  if (first >= Mp) return;
+  const int p0 = (int)first, p1 = Mp - p0 < per ? Mp : p0 + per;
+  // groups of up to 64 probes: resolved PROBE_ROWS of one node at a time into the wave's
   // LDS row (entry q: probe g0 + q's agent and node, its state word and index in the
   // node), then every lane claims its own at once.  The node's data is reloaded per
   // group and the row is in LDS, so neither is held in registers through the other
   // phase (more wavefronts resident)
   __shared__ uint4 s_res[WG / 64][64];
-  uint4* res = s_res[threadIdx.x >> 6];
-  for (int64_t g0 = p0; g0 < p1; g0 += 64) {
-    const int64_t g1 = g0 + 64 < p1 ? g0 + 64 : p1;
-    int node = -1, ns = 0, stile = 0, sntile = 0;   // lane l: span l of the node (first tile, tiles)
-    int64_t node_lo = 0, node_hi = 0, W = 0, spx = INT64_MAX;
+  uint4* res = s_res[wave];
+  for (int g0 = p0; g0 < p1; g0 += 64) {
+    const int g1 = p1 - g0 < 64 ? p1 : g0 + 64;
+    int node = -1, ns = 0, s0 = 0, stile = 0, sntile = 0;   // lane l: span l of the node (first tile, tiles)
+    int node_lo = 0, node_hi = 0;
+    int64_t W = 0, spx = INT64_MAX;
     uint64_t seed = 0;
     uint32_t lnode = 0;
-    for (int64_t p = g0; p < g1; ++p) {
+    for (int p = g0; p < g1;) {
       if (node < 0 || p >= node_hi) {
         node = __builtin_amdgcn_readfirstlane((int)find_node(off, N, p));
-        node_lo = off[node];
-        node_hi = off[node + 1];
+        node_lo = __builtin_amdgcn_readfirstlane((int)off[node]);
+        node_hi = __builtin_amdgcn_readfirstlane((int)off[node + 1]);
         const NodeInfo& ni = d.ninfo[node];
         const SpanLane sl = d.span_lane[(size_t)node * 64 + lane];   // beside the NodeInfo loads
         seed = ni.seed;
         lnode = (uint32_t)ni.lnode;
         W = d.W_round[node];
         ns = ni.n_spans;
+        s0 = ni.span_begin;
         spx = ns <= 64 ? sl.prefix : INT64_MAX;
         stile = sl.tile0;
         sntile = sl.ntiles;
       }
-      const int64_t j = p - node_lo;
+      // up to PROBE_ROWS probes of the node, one per row
+      const int left = (node_hi < g1 ? node_hi : g1) - p;
+      const int np = left < PROBE_ROWS ? left : PROBE_ROWS;
+      const int row = lane >> 4;
+      const int j = p - node_lo + row;
       const uint4 o = philox((uint32_t)j, lnode, (uint32_t)t, ST_PROBE | (1u << 8), seed);
       const uint64_t u = (uint64_t)o.x | ((uint64_t)o.y << 32);
       const int64_t T = (int64_t)mulhi64(u, (uint64_t)(W > 0 ? W : 0));
       int64_t slot = -1;
       uint32_t word = 0;
       if (W > 0) {
-        if (ns <= 64) {
-          const uint64_t ok = __ballot(spx <= T);      // monotone over the node's spans
-          if (ok) {
-            const int L = 63 - __clzll((unsigned long long)ok);
-            slot = resolve_in_tiles<false, true>(d, __shfl(stile, L, 64), __shfl(sntile, L, 64), __shfl(spx, L, 64),
-                                                 T, lane, &word);
-          }
-        } else {
-          slot = resolve_probe<false, true>(d, node, T, d.span_prefix, lane, &word);
-        }
+        const RowSpan rs = row_spans<false>(d, np, T, ns, s0, spx, stile, sntile, d.span_prefix, lane);
+        slot = resolve_row<false, true>(d, rs.tile0, rs.ntiles, rs.base, T, lane, word);
       }
-      if (lane == 0) {
-        const uint64_t e = (slot < 0 ? SEL_SLOT : (uint64_t)slot) | ((uint64_t)node << 40);
-        res[p - g0] = make_uint4((uint32_t)e, (uint32_t)(e >> 32), word, (uint32_t)j);
+      // the lane that holds the row's agent writes the probe's entry, lane 0 of the row
+      // that of a probe without one
+      const bool hit = slot >= 0;
+      const uint32_t hb = (uint32_t)(__ballot(hit) >> (lane & 48)) & 0xffffu;
+      if (row < np && (hit || (hb == 0 && (lane & 15) == 0))) {
+        const uint64_t e = (hit ? (uint64_t)slot : SEL_SLOT) | ((uint64_t)node << 40);
+        res[p - g0 + row] = make_uint4((uint32_t)e, (uint32_t)(e >> 32), word, (uint32_t)j);
       }
+      p += np;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -3248,7 +3362,7 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
       my_j = r.w;
     }
     // the group's claims, lane q for probe g0 + q
-    const int64_t p = g0 + lane;
+    const int p = g0 + lane;
     int k = -1;
     bool won = false;
     uint4 rec = make_uint4(0u, 0u, 0u, 0u);
@@ -3269,7 +3383,7 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
         }
         rec = d.rec[my_slot];   // the entry's record fields do not change when an agent is exposed
         w = weight_q24(d.risk[my_slot]);
-        if (claim_from(d.state, my_slot, my_word)) {   // the first probe of an agent claims it
+        if (claim_from(d.state, my_slot, my_word, SEL_MARK)) {   // the first probe of an agent claims it
           won = true;
           k = strain_draw(d, thr, ni.seed, ni.slot_base, my_slot, t);
           *rec_byte(d, my_slot, RB_STRAIN) = (int8_t)k;
@@ -3277,29 +3391,14 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
       } else {
         atomicOr(d.err, ERR_SAMPLING);
       }
-      d.sel_list[base + p] = (my_slot < 0 ? SEL_SLOT : (uint64_t)my_slot) | ((uint64_t)my_node << 40) | (won ? SEL_WON : 0);
+      // k_finish counts the node's winners by strain
+      d.sel_list[base + p] = (my_slot < 0 ? SEL_SLOT : (uint64_t)my_slot) |
+                             (won ? SEL_WON | ((uint64_t)k << SEL_STRAIN) : 0);
       if (won) d.sel_word[base + p] = w < (int64_t)0xFFFFFFFF ? (uint32_t)w : 0xFFFFFFFFu;   // k_finish removes it
     }
-    const int wn = won ? my_node : -1;
     const uint4 ent = won ? exposed_entry_rec(my_slot, rec, k, t, r0_sel(r0v, k)) : make_uint4(0u, 0u, 0u, 0u);
     if (at) *at = ent;
-    // new exposures by strain: one atomic per strain when the group's winners share a node
-    const int n0 = __shfl(wn, __ffsll((unsigned long long)__ballot(wn >= 0)) - 1, 64);
-    const bool same = __ballot(wn >= 0 && wn != n0) == 0;
-    if (same) {
-      const uint64_t any = __ballot(wn >= 0);
-      if (any) {
-        for (int s = 0; s < d.K; ++s) {
-          const int c = __popcll(__ballot(k == s));
-          if (lane == 0 && c) atomicAdd(d.newexp + n0 * LP_MAX_STRAINS + s, c);
-        }
-        if (lane == 0) atomicAdd(d.n_uniq + n0, __popcll(any));
-      }
-    } else if (wn >= 0) {
-      atomicAdd(d.newexp + wn * LP_MAX_STRAINS + k, 1);
-      atomicAdd(d.n_uniq + wn, 1);
-    }
-    if (won && !at) append_entry(d, nxt, wn, ent);
+    if (won && !at) append_entry(d, nxt, my_node, ent);
   }
 }
 
@@ -3311,111 +3410,159 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
 // L2 (agent-scope atomics, atomic loads and stores), so __syncthreads (workgroup-
 // scope release / acquire) orders them: a device-scope fence would also write back
 // the XCD's whole L2, at a cost of microseconds.
+// What bounds it is the latency of the probes (2.5 us a step of PROBE_ROWS per wavefront:
+// two dependent loads and about 500 instructions), so a node gets as many wavefronts as
+// stay resident: 1024 threads up to one node per CU, else 512 held to 6 waves per SIMD.
+// Years with 256 / 512 / 1024 threads a node: 14 nodes 28.2 / 26.7 / 25.9 ms, 64
+// replicates (1530 nodes) 82.0 / 76.2 / 74.5 ms, national (774 nodes) 39.6 / 40.0 / 41.0
+// ms.  The node's span weights, list length and exposure counts stay in LDS between rounds
+// and leave once at the end; the winners of round 1 are counted here, from their entries,
+// because k_sample's atomics on one node's counters serialised (14-node year 25.9 -> 23.4
+// ms without them).
 constexpr int FIN_LDS = 2048;
-__global__ void __launch_bounds__(WG) k_finish(Dev d) {
+template <int NT, int MINW>
+__global__ void __launch_bounds__(NT, MINW) k_finish(Dev d) {
   const int4 dy = today(d);
   const int32_t t = dy.x;
   const int n = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // the same in the wave's lanes
   __shared__ int64_t sh_base;
   __shared__ uint64_t s_sel[FIN_LDS];        // a round's selected entries when they fit
   __shared__ int32_t s_ne[LP_MAX_STRAINS];   // the node's new exposures by strain (one global add each)
   __shared__ int32_t s_claimed;
-  // most nodes have nothing left after round 1: one round of loads decides
-  const int32_t size = d.size[n], take_all = d.take_all[n], uniq0 = d.n_uniq[n], m1 = d.m_round[n];
-  const bool later = size > 0 && (take_all || size - uniq0 > 0);
+  __shared__ int32_t s_cnt;                  // length of the node's list for tomorrow, which only this workgroup extends
+  __shared__ int64_t s_spw[64];              // up to 64 spans: weight that left each span, not yet in its partial
+  __shared__ int64_t s_w[64];                // and the weight each span has left
+  const int32_t size = d.size[n], take_all = d.take_all[n], m1 = d.m_round[n];
+  if (size <= 0) return;
   const NodeInfo& ni = d.ninfo[n];
+  const int nxt = (t + 1) & 1;
+  const bool lane_spans = ni.n_spans <= 64;
+  const int64_t tile0 = ni.seg_begin / LP_TILE;
+  // what the later rounds start from loads beside round 1's entries: lane l of every wave
+  // holds span l's tiles, thread l its weight at the round's start
+  SpanLane sl{INT64_MAX, 0, 0};
+  int64_t w_node = 0;
+  if (lane_spans) {
+    sl = d.span_lane[(size_t)n * 64 + lane];
+    w_node = d.W_round[n];
+  }
+  const int32_t cnt0 = d.ei_cnt[(size_t)nxt * d.n_nodes + n];
+  uint64_t thr[LP_MAX_STRAINS];   // the node's cumulative strain thresholds
+#pragma unroll
+  for (int q = 0; q < LP_MAX_STRAINS; ++q) thr[q] = d.thr_strain[(size_t)n * LP_MAX_STRAINS + q];
+  if (tid < 64) s_spw[tid] = 0;
+  if (tid < LP_MAX_STRAINS) s_ne[tid] = 0;
+  if (tid == 0) { s_claimed = 0; s_cnt = cnt0; }
   // (a round 1 that overflowed the selected list ran no probes: probe_off[N] = 0)
   if (m1 > 0 && d.probe_off[d.n_nodes] > 0) {
-    // round 1's winners (claimed by k_sample, state SEL_MARK): E now, and their weights
-    // leave the chunk and span sums before any later round reads them
-    // eight entries per thread with their loads in flight together; up to 64 spans the
+    // round 1's winners (claimed by k_sample, state SEL_MARK): E now, counted by strain, and
+    // their weights leave the chunk and span sums before any later round reads them.
+    // Eight entries per thread with their loads in flight together; up to 64 spans the
     // span weights are summed in LDS and leave with one atomic per span
-    __shared__ int64_t s_spw[64];
-    const bool lds_spans = ni.n_spans <= 64;
-    if (tid < 64) s_spw[tid] = 0;
     __syncthreads();
     const int64_t b1 = d.round_base[1] + d.probe_off[n];
-    const int64_t tile0 = ni.seg_begin / LP_TILE;
     constexpr int U = 8;
-    for (int j0 = 0; j0 < m1; j0 += U * WG) {
+    for (int j0 = 0; j0 < m1; j0 += U * NT) {
       uint64_t e[U];
       uint32_t wq[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int j = j0 + u * WG + tid;
+        const int j = j0 + u * NT + tid;
         e[u] = j < m1 ? d.sel_list[b1 + j] : 0ull;
         wq[u] = j < m1 ? d.sel_word[b1 + j] : 0u;
       }
+      uint64_t c_k = 0;   // winners by strain, 16 bits each (at most 64 * U in a wave)
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (!(e[u] & SEL_WON)) continue;
         const int64_t slot = (int64_t)(e[u] & SEL_SLOT);
+        c_k += 1ull << (16 * ((e[u] >> SEL_STRAIN) & (LP_MAX_STRAINS - 1)));
         const int64_t w = wq[u] != 0xFFFFFFFFu ? (int64_t)wq[u] : weight_q24(d.risk[slot]);
         d.state[slot] = 1;
         const unsigned long long dw = (unsigned long long)(-w);
         atomicAdd(reinterpret_cast<unsigned long long*>(d.chunk_sum + (slot >> 8)), dw);
         const int ls = (int)((slot / LP_TILE - tile0) >> d.tpw_sh);   // the node's span
-        if (lds_spans) atomicAdd(reinterpret_cast<unsigned long long*>(&s_spw[ls]), dw);
+        if (lane_spans) atomicAdd(reinterpret_cast<unsigned long long*>(&s_spw[ls]), dw);
         else atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(ni.span_begin + ls) * NPART + P_SW), dw);
       }
+      c_k = (uint64_t)wave_sum_i64((int64_t)c_k);
+      const int c = lane < LP_MAX_STRAINS ? (int)((c_k >> (16 * lane)) & 0xffffu) : 0;
+      if (c) { atomicAdd(&s_ne[lane], c); atomicAdd(&s_claimed, c); }
     }
     __syncthreads();
-    if (lds_spans && tid < ni.n_spans && s_spw[tid] != 0)
-      atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(ni.span_begin + tid) * NPART + P_SW),
-                (unsigned long long)s_spw[tid]);
-    if (!later) return;
-    __syncthreads();   // the weights and states before the later rounds
-  } else if (!later) {
-    return;
+    // most nodes have nothing left after round 1
+    if (s_claimed >= size) {
+      if (lane_spans && tid < ni.n_spans && s_spw[tid] != 0)
+        atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(ni.span_begin + tid) * NPART + P_SW),
+                  (unsigned long long)s_spw[tid]);
+      if (tid < LP_MAX_STRAINS) d.newexp[n * LP_MAX_STRAINS + tid] = s_ne[tid];
+      return;
+    }
   }
-  if (tid < LP_MAX_STRAINS) s_ne[tid] = 0;
-  if (tid == 0) s_claimed = 0;
-  uint64_t thr[LP_MAX_STRAINS];   // the node's cumulative strain thresholds, loaded once
   float r0v[LP_MAX_STRAINS];
 #pragma unroll
-  for (int q = 0; q < LP_MAX_STRAINS; ++q) {
-    thr[q] = d.thr_strain[(size_t)n * LP_MAX_STRAINS + q];
-    r0v[q] = ni.r0k[q];
+  for (int q = 0; q < LP_MAX_STRAINS; ++q) r0v[q] = ni.r0k[q];
+  if (lane_spans && tid < 64) {
+    const int64_t after = __shfl_down(sl.prefix, 1, 64);
+    s_w[tid] = tid < ni.n_spans ? (tid == ni.n_spans - 1 ? w_node : after) - sl.prefix + s_spw[tid] : 0;
   }
-  __syncthreads();
-  const int nxt = (t + 1) & 1;
+  __syncthreads();   // the weights and states before the later rounds
+  uint4* list = d.ei_list + (size_t)nxt * (size_t)d.capacity + ni.seg_begin;
+  // appends the entries of the lanes with `flag` (every lane of the wave calls)
+  auto append = [&](bool flag, const uint4& e) {
+    const uint64_t mk = __ballot(flag);
+    if (mk == 0) return;
+    int base = 0;
+    if (lane == 0) base = atomicAdd(&s_cnt, __popcll(mk));
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (flag) list[base + __popcll(mk & ((1ull << lane) - 1ull))] = e;
+  };
+  // an agent that becomes E leaves its chunk's weight and its span's
+  auto leave = [&](int64_t slot, int64_t w) {
+    if (lane_spans) {
+      const unsigned long long dw = (unsigned long long)(-w);
+      atomicAdd(reinterpret_cast<unsigned long long*>(d.chunk_sum + (slot >> 8)), dw);
+      const int ls = (int)((slot / LP_TILE - tile0) >> d.tpw_sh);
+      atomicAdd(reinterpret_cast<unsigned long long*>(&s_w[ls]), dw);
+      atomicAdd(reinterpret_cast<unsigned long long*>(&s_spw[ls]), dw);
+    } else {
+      unweight_in(d, span_of(d, n, slot), slot, w);
+    }
+  };
   if (take_all) {
     const int64_t lo = ni.seg_begin, hi = d.live_end[n];
-    for (int64_t i0 = lo; i0 < hi; i0 += WG) {         // uniform trip count: whole waves append
+    for (int64_t i0 = lo; i0 < hi; i0 += NT) {         // uniform trip count: whole waves append
       const int64_t i = i0 + tid;
       bool ex = false;
       int kx = 0;
       uint4 rec = make_uint4(0u, 0u, 0u, 0u);
-      if (i < hi && d.state[i] == 0 && weight_q24(d.risk[i]) > 0) {
-        rec = d.rec[i];
-        unweight(d, n, i);
-        kx = expose_agent_thr(d, thr, ni.seed, ni.slot_base, i, t);
-        atomicAdd(&s_ne[kx], 1);
-        ex = true;
+      if (i < hi && d.state[i] == 0) {
+        const int64_t w = weight_q24(d.risk[i]);
+        if (w > 0) {
+          rec = d.rec[i];
+          leave(i, w);
+          kx = expose_agent_thr(d, thr, ni.seed, ni.slot_base, i, t);
+          atomicAdd(&s_ne[kx], 1);
+          ex = true;
+        }
       }
-      wave_append_entry(d, nxt, n, ex ? exposed_entry_rec(i, rec, kx, t, r0_sel(r0v, kx)) : make_uint4(0u, 0u, 0u, 0u),
-                        ex, lane);
+      append(ex, ex ? exposed_entry_rec(i, rec, kx, t, r0_sel(r0v, kx)) : make_uint4(0u, 0u, 0u, 0u));
     }
   } else {
     const int s0 = ni.span_begin, s1 = ni.span_begin + ni.n_spans;
-    // up to 64 spans: lane l of every wave holds span l's tile range and, each round,
-    // its prefix of the remaining weights (a wave scan of the span partials)
-    const bool lane_spans = ni.n_spans <= 64;
-    const bool my_span = lane_spans && lane < ni.n_spans;
-    const int4 sp4 = my_span ? d.spans[s0 + lane] : make_int4(0, 0, 0, 0);
     for (int round = 2;; ++round) {
       if (round > MAX_ROUNDS) { if (tid == 0) atomicOr(d.err, ERR_SAMPLING); break; }
-      const int32_t need = size - (uniq0 + s_claimed);
+      const int32_t need = size - s_claimed;
       if (need <= 0) break;
+      // the remaining weight and, lane = span, its prefix
       int64_t W, spx = INT64_MAX;
       if (lane_spans) {
-        const int64_t v = my_span ? __hip_atomic_load(d.partials + (size_t)(s0 + lane) * NPART + P_SW, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT)
-                                  : 0;
+        const int64_t v = s_w[lane];
         const int64_t incl = wave_incl_scan_i64(v);
-        W = __shfl(incl, 63, 64);
-        if (my_span) spx = incl - v;
+        W = readlane_i64(incl, 63);
+        if (lane < ni.n_spans) spx = incl - v;
       } else {
         W = node_span_scan<true>(d.partials, d.fin_prefix, s0, s1);
       }
@@ -3423,82 +3570,77 @@ __global__ void __launch_bounds__(WG) k_finish(Dev d) {
       // a round of up to FIN_LDS probes keeps them in LDS; a larger one reserves space in
       // the selected list (uniform over the workgroup)
       const bool in_lds = need <= FIN_LDS;
-      if (tid == 0) {
-        int64_t b = 0;
-        if (!in_lds) {
-          b = atomicAdd(reinterpret_cast<unsigned long long*>(d.sel_count), (unsigned long long)need);
+      uint64_t* gsel = nullptr;
+      if (!in_lds) {
+        if (tid == 0) {
+          int64_t b = atomicAdd(reinterpret_cast<unsigned long long*>(d.sel_count), (unsigned long long)need);
           if (b + need > d.sel_cap) {
             atomicOr(d.err, ERR_OVERFLOW);
             b = -1;
           }
+          sh_base = b;
         }
-        sh_base = b;
+        __syncthreads();
+        if (sh_base < 0) break;
+        gsel = d.sel_list + sh_base;
       }
-      __syncthreads();
-      const int64_t base = sh_base;
-      if (base < 0) break;
-      uint64_t* gsel = d.sel_list + base;
-      for (int j = wave; j < need; j += WG / 64) {
+      for (int j0 = wave * PROBE_ROWS; j0 < need; j0 += NT / 64 * PROBE_ROWS) {   // PROBE_ROWS probes per wave
+        const int np = need - j0 < PROBE_ROWS ? need - j0 : PROBE_ROWS;
+        const int row = lane >> 4, j = j0 + row;
         const uint4 o = philox((uint32_t)j, (uint32_t)ni.lnode, (uint32_t)t,
                                ST_PROBE | ((uint32_t)round << 8), ni.seed);
         const uint64_t u = (uint64_t)o.x | ((uint64_t)o.y << 32);
         const int64_t T = (int64_t)mulhi64(u, (uint64_t)W);
-        int64_t slot = -1;
-        if (lane_spans) {
-          const uint64_t ok = __ballot(spx <= T);         // monotone over the node's spans
-          if (ok) {
-            const int L = 63 - __clzll((unsigned long long)ok);
-            slot = resolve_in_tiles<true, false>(d, __shfl(sp4.y, L, 64), __shfl(sp4.z, L, 64), __shfl(spx, L, 64), T,
-                                          lane);
-          }
-        } else {
-          slot = resolve_probe<true, false>(d, n, T, d.fin_prefix, lane);
-        }
-        if (lane == 0) {
-          const uint64_t e = slot < 0 ? SEL_INVALID : ((uint64_t)slot | ((uint64_t)n << 40));
-          if (slot < 0) atomicOr(d.err, ERR_SAMPLING);
+        uint32_t word = 0;
+        const RowSpan rs = row_spans<true>(d, np, T, ni.n_spans, s0, spx, sl.tile0, sl.ntiles, d.fin_prefix, lane);
+        const int64_t slot = resolve_row<true, false>(d, rs.tile0, rs.ntiles, rs.base, T, lane, word);
+        const bool hit = slot >= 0;
+        const uint32_t hb = (uint32_t)(__ballot(hit) >> (lane & 48)) & 0xffffu;
+        if (row < np && (hit || (hb == 0 && (lane & 15) == 0))) {
+          // slots fit 32 bits (capacity below 2^32): the agent and its state word as read
+          const uint64_t e = hit ? ((uint64_t)slot | ((uint64_t)word << 32)) : SEL_INVALID;
+          if (!hit) atomicOr(d.err, ERR_SAMPLING);
           if (in_lds) s_sel[j] = e;
           else __hip_atomic_store(gsel + j, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
       }
       __syncthreads();
-      for (int j = tid; j < need; j += WG) {
-        const uint64_t e = in_lds ? s_sel[j] : __hip_atomic_load(gsel + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (e == SEL_INVALID) continue;
-        const int64_t slot = (int64_t)(e & ((1ull << 40) - 1));
-        if (claim(d.state, slot)) {
-          unweight(d, n, slot);
-          atomicAdd(&s_claimed, 1);
-        } else if (in_lds) {
-          s_sel[j] = SEL_INVALID;
-        } else {
-          __hip_atomic_store(gsel + j, SEL_INVALID, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-      __syncthreads();   // the claims and weight updates before the exposures and the next round
-      for (int j0 = 0; j0 < need; j0 += WG) {          // uniform trip count: whole waves append
+      // every probe of the round is resolved: the first probe of an agent makes it E at
+      // once (claim, weights, strain and list entry in one pass, everything it reads in
+      // flight with the claim)
+      for (int j0 = 0; j0 < need; j0 += NT) {          // uniform trip count: whole waves append
         const int j = j0 + tid;
         const uint64_t e = j >= need ? SEL_INVALID
                            : in_lds ? s_sel[j]
                                     : __hip_atomic_load(gsel + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const int64_t slot = (int64_t)(e & ((1ull << 40) - 1));
-        const bool ex = e != SEL_INVALID;
+        const int64_t slot = (int64_t)(uint32_t)e;
+        bool ex = e != SEL_INVALID;
         int kx = 0;
         uint4 rec = make_uint4(0u, 0u, 0u, 0u);
         if (ex) {
           rec = d.rec[slot];
-          kx = expose_agent_thr(d, thr, ni.seed, ni.slot_base, slot, t);
-          atomicAdd(&s_ne[kx], 1);
+          const float rk = d.risk[slot];
+          ex = claim_from(d.state, slot, (uint32_t)(e >> 32), 1);
+          if (ex) {
+            leave(slot, weight_q24(rk));
+            kx = strain_draw(d, thr, ni.seed, ni.slot_base, slot, t);
+            *rec_byte(d, slot, RB_STRAIN) = (int8_t)kx;
+            atomicAdd(&s_ne[kx], 1);
+          }
         }
-        wave_append_entry(d, nxt, n, ex ? exposed_entry_rec(slot, rec, kx, t, r0_sel(r0v, kx)) : make_uint4(0u, 0u, 0u, 0u),
-                          ex, lane);
+        const uint64_t won = __ballot(ex);
+        if (lane == 0 && won) atomicAdd(&s_claimed, __popcll(won));
+        append(ex, ex ? exposed_entry_rec(slot, rec, kx, t, r0_sel(r0v, kx)) : make_uint4(0u, 0u, 0u, 0u));
       }
-      __syncthreads();
+      __syncthreads();   // the claims and weight updates before the next round
     }
   }
   __syncthreads();
-  if (tid < LP_MAX_STRAINS && s_ne[tid]) atomicAdd(d.newexp + n * LP_MAX_STRAINS + tid, s_ne[tid]);
-  if (tid == 0 && s_claimed) atomicAdd(d.n_uniq + n, s_claimed);
+  if (lane_spans && tid < ni.n_spans && s_spw[tid] != 0)
+    atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(ni.span_begin + tid) * NPART + P_SW),
+              (unsigned long long)s_spw[tid]);
+  if (tid < LP_MAX_STRAINS) d.newexp[n * LP_MAX_STRAINS + tid] = s_ne[tid];
+  if (tid == 0 && s_cnt != cnt0) d.ei_cnt[(size_t)nxt * d.n_nodes + n] = s_cnt;
 }
 
 // Per node: transmission incidence and the log rows of day t, in two parts as
