@@ -105,7 +105,6 @@ struct lp_ctx {
   int32_t agent_grid = 1;
   int32_t ei_grid = 2048, sample_grid = 2048;     // launch shapes of the list pass and the sampler
   bool finish_wide = false;                       // k_finish with 1024 threads a node (no more nodes than CUs)
-  bool mix_wide = false;                          // k_mix_foi<4> (more nodes than resident waves)
   int32_t mix_tiles = 0;                           // mix_mode 1: 16-row tiles of the largest simulation
   std::vector<void*> allocs;
   // per day kind (plain, FULL_* combinations, their list forms): graph[kind][j] runs 2^j
@@ -344,10 +343,7 @@ int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool ad
   if (mask & LP_STAGE_TRANSMISSION) {
     if (c->cfg.mix_mode == 1)
       hipLaunchKernelGGL(lp::k_mix_mfma, dim3(c->cfg.n_sims, c->mix_tiles), dim3(64), 0, s, d);
-    if (c->mix_wide)
-      hipLaunchKernelGGL(lp::k_mix_foi<4>, dim3(grid_of(N, lp::WG / 64)), dim3(lp::WG), 0, s, d, mask);
-    else
-      hipLaunchKernelGGL(lp::k_mix_foi<1>, dim3(grid_of(N, lp::WG / 64)), dim3(lp::WG), 0, s, d, mask);
+    hipLaunchKernelGGL(lp::k_mix_foi, dim3(grid_of(N, lp::MIX_ROWS)), dim3(lp::WG), 0, s, d, mask);
     // with the probe offsets in LDS k_sample plans round 1 itself
     const size_t off_lds = (N + 1 <= lp::LDS_OFF_MAX) ? (size_t)(N + 1) * sizeof(int64_t) : 0;
     if (!off_lds) hipLaunchKernelGGL(lp::k_plan, dim3(1), dim3(lp::WG), 0, s, d, 1);
@@ -528,13 +524,9 @@ int lp_prepare(lp_ctx* c) {
     const size_t off_lds = (N + 1 <= lp::LDS_OFF_MAX) ? (size_t)(N + 1) * sizeof(int64_t) : 0;
     if (!c->cfg.ei_grid) c->ei_grid = resident(reinterpret_cast<const void*>(lp::k_ei), 0, kEiGrid);
     if (!c->cfg.sample_grid) c->sample_grid = resident(reinterpret_cast<const void*>(lp::k_sample), off_lds, kSampleGrid);
-    // k_mix_foi: the variant held to 4 waves per SIMD once its workgroups outnumber those
-    // of the unrestricted variant resident at once
-    const int mix_blocks = (int)grid_of(N, lp::WG / 64);
     // k_finish: 1024 threads a node while every node's workgroup is resident at once (one a
     // CU); above that 512 threads held to 6 waves per SIMD (three a CU)
     c->finish_wide = N <= cus;
-    c->mix_wide = mix_blocks > resident(reinterpret_cast<const void*>(lp::k_mix_foi<1>), 0, 1 << 30);
   }
   int4* spans_d; int32_t* nspan_d;
   int rc;

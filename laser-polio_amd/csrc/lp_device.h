@@ -173,7 +173,7 @@ __device__ __forceinline__ float log1pf_lp(float x) {
 // to).  Integer results do not depend on the order.  The scans sit on the day kernels'
 // chains of dependent steps: the 14-node year went from 42.4 to 39.9 ms, a batch of 64
 // simulations from 115.5 to 108.3 ms a year, the national year from 39.5 to 38.4 ms.
-constexpr int DPP_ROW_SHR = 0x110, DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143;
+constexpr int DPP_ROW_SHL = 0x100, DPP_ROW_SHR = 0x110, DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143;
 
 // The source lane's v, or `old` on lanes without a source lane or outside row_mask.
 template <int CTRL, int ROW_MASK>
@@ -190,6 +190,23 @@ __device__ __forceinline__ int64_t readlane_i64(int64_t v, int lane) {
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int32_t)(uint32_t)v, lane);
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int32_t)(v >> 32), lane);
   return (int64_t)(((uint64_t)hi << 32) | lo);
+}
+
+// x plus the value N lanes up in the row (lanes without one keep x).
+template <int N>
+__device__ __forceinline__ float add_row_shl(float x) {
+  return x + __builtin_bit_cast(float, dpp_i32<DPP_ROW_SHL | N, 0xf>(0, __builtin_bit_cast(int32_t, x)));
+}
+// The halving-tree sum of the 64 lanes' x (x[l] + x[l + 32], then + 16, 8, 4, 2, 1), in
+// every lane.
+__device__ __forceinline__ float wave_tree_sum_f32(float x) {
+  x = x + __shfl_down(x, 32, 64);
+  x = x + __shfl_down(x, 16, 64);
+  x = add_row_shl<8>(x);
+  x = add_row_shl<4>(x);
+  x = add_row_shl<2>(x);
+  x = add_row_shl<1>(x);
+  return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int32_t, x)));
 }
 
 // Inclusive prefix sum inside each row of 16 lanes.

@@ -2660,12 +2660,6 @@ __device__ void plan_scan(const Dev& d, int round) {
 }
 
 // ---------------------------------------------------------------------------
-// One wavefront per node.  The network mix sum_j N_ji beta_j is added in the
-// order of a 256-lane strided sum followed by a halving tree over the 256
-// partials: lane l holds the partials of lanes l, l + 64, l + 128, l + 192, folds
-// them in-lane for the first two tree levels and across lanes for the rest.
-// `off`: no transmission today (the node's sampling sizes are zeroed instead); a
-// stopped simulation is tested after the mix's loads are issued.
 // t / s, correctly rounded, for a step number s <= 64 that is the same on every lane:
 // t * y with y = RN(1/s) (lane s - 1 of ystep), refined by its exact residual
 // r = t - s * (t * y) (Markstein's correction).  Over every significand of t and
@@ -2679,13 +2673,84 @@ __device__ __forceinline__ float step_quot(float t, int s, float ystep) {
   return __builtin_fmaf(r, y, q0);
 }
 
-__device__ void mix_foi_node(const Dev& d, int i, const NodeInfo& ni, int32_t t, int lane, bool off) {
+// The network mix sum_j N_ji beta_j of the MIX_ROWS consecutive nodes of a workgroup, one
+// per wavefront afterwards.  Each node's sum is added in the order of a 256-lane strided
+// sum followed by a halving tree over the 256 partials, the oracle's order.  Thread p
+// holds partial p of all MIX_ROWS nodes, so a source's weights (16 bytes, four strains)
+// load once for MIX_ROWS network rows: a wavefront per node read four times the
+// network's bytes again in weights (5000 nodes: 62 us a day, 100 MB of network rows
+// and 400 MB of weights; 150 days of the continental workload went from 39.2 to 33.7 ms,
+// up to 1000 nodes nothing changed).  The first two tree levels pair partials of different
+// wavefronts: they meet in LDS (part), from where wavefront w takes node w's.
+constexpr int MIX_ROWS = WG / 64;
+constexpr int MIX_U = 4;          // sources per thread in flight: 1024 sources of the workgroup
+
+__device__ __forceinline__ void mix_rows(const Dev& d, int i0, float (*part)[MIX_ROWS][LP_MAX_STRAINS][64]) {
+  const int tid = threadIdx.x, N = d.n_nodes;
+  const float* NT[MIX_ROWS];
+  const float4* B[MIX_ROWS];
+  int ns[MIX_ROWS];
+  bool one_sim = true;
+#pragma unroll
+  for (int q = 0; q < MIX_ROWS; ++q) {
+    const NodeInfo& ni = d.ninfo[i0 + q < N ? i0 + q : N - 1];   // past the last node: its row again, unused
+    ns[q] = ni.sim_nodes;
+    NT[q] = d.network_t + ni.net_off + (size_t)ni.lnode * ns[q];
+    B[q] = reinterpret_cast<const float4*>(d.beta_f) + ni.sim_node_begin;
+    one_sim = one_sim && B[q] == B[0] && ns[q] == ns[0];
+  }
+  float acc[MIX_ROWS][LP_MAX_STRAINS];
+#pragma unroll
+  for (int q = 0; q < MIX_ROWS; ++q) {
+#pragma unroll
+    for (int k = 0; k < LP_MAX_STRAINS; ++k) acc[q][k] = 0.0f;
+  }
+  auto add = [&](int q, float nt, const float4& b) {
+    acc[q][0] = __builtin_fmaf(nt, b.x, acc[q][0]);
+    acc[q][1] = __builtin_fmaf(nt, b.y, acc[q][1]);
+    acc[q][2] = __builtin_fmaf(nt, b.z, acc[q][2]);
+    acc[q][3] = __builtin_fmaf(nt, b.w, acc[q][3]);
+  };
+  if (one_sim) {                                          // uniform
+    for (int j0 = tid; j0 < ns[0]; j0 += MIX_U * WG) {
+      float nt[MIX_U][MIX_ROWS];
+      float4 b[MIX_U];
+#pragma unroll
+      for (int u = 0; u < MIX_U; ++u) {
+        const int j = j0 + u * WG;
+        const bool v = j < ns[0];
+        b[u] = v ? B[0][j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+        for (int q = 0; q < MIX_ROWS; ++q) nt[u][q] = v ? NT[q][j] : 0.0f;
+      }
+#pragma unroll
+      for (int u = 0; u < MIX_U; ++u) {
+        if (j0 + u * WG >= ns[0]) break;
+#pragma unroll
+        for (int q = 0; q < MIX_ROWS; ++q) add(q, nt[u][q], b[u]);
+      }
+    }
+  } else {                                                // a batch: nodes of different simulations
+#pragma unroll
+    for (int q = 0; q < MIX_ROWS; ++q)
+      for (int j = tid; j < ns[q]; j += WG) add(q, NT[q][j], B[q][j]);
+  }
+#pragma unroll
+  for (int q = 0; q < MIX_ROWS; ++q) {
+#pragma unroll
+    for (int k = 0; k < LP_MAX_STRAINS; ++k) part[tid >> 6][q][k][tid & 63] = acc[q][k];
+  }
+}
+
+// Node i's force of infection and count draw (one wavefront, w of its workgroup), from the
+// workgroup's mix partials.  `off`: no transmission today (the node's sampling sizes are
+// zeroed instead); not `on`: a wavefront past the last node, here for the barrier only.
+__device__ void mix_foi_node(const Dev& d, int i, const NodeInfo& ni, int32_t t, int lane, int w, bool off,
+                             const float (*mix)[MIX_ROWS][LP_MAX_STRAINS][64], bool on) {
   const int K = d.K;
   const int sim = ni.sim;
-  const int ns = ni.sim_nodes, li = ni.lnode;
-  const float* NT = d.network_t + ni.net_off + (size_t)li * ns;
-  const float4* B = reinterpret_cast<const float4*>(d.beta_f) + ni.sim_node_begin;
-  // the node's own inputs, loaded ahead of the mix
+  const int li = ni.lnode;
+  // the node's own inputs
   const int64_t* tl = d.node_tally + (size_t)i * NPART;
   int32_t* lcnt = d.ei_cnt + (size_t)((t + 1) & 1) * d.n_nodes + i;   // tomorrow's list (its passes ran)
   const int32_t lbase = *lcnt;
@@ -2697,57 +2762,21 @@ __device__ void mix_foi_node(const Dev& d, int i, const NodeInfo& ni, int32_t t,
 #pragma unroll
   for (int k = 0; k < LP_MAX_STRAINS; ++k) ibk[k] = k < K ? tl[P_IB0 + k] : 0;
   const int64_t sw = tl[P_SW], scnt = tl[P_S], spos = tl[P_SPOS];
-  // lane l's partial of group v sums sources j = l + 64 v + 256 r for r = 0, 1, ...;
-  // the sources below MIX_PRE * 64 are loaded together first
-  constexpr int MIX_PRE = 16;
-  float ntv[MIX_PRE];
-  float4 bv[MIX_PRE];
-#pragma unroll
-  for (int m = 0; m < MIX_PRE; ++m) {
-    const int j = lane + 64 * m;
-    ntv[m] = j < ns ? NT[j] : 0.0f;
-    bv[m] = j < ns ? B[j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  }
-  float acc[4][LP_MAX_STRAINS];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-#pragma unroll
-    for (int k = 0; k < LP_MAX_STRAINS; ++k) acc[v][k] = 0.0f;
-  }
-#pragma unroll
-  for (int m = 0; m < MIX_PRE; ++m) {
-    const int v = m & 3;
-    if (lane + 64 * m < ns) {
-      acc[v][0] = __builtin_fmaf(ntv[m], bv[m].x, acc[v][0]);
-      acc[v][1] = __builtin_fmaf(ntv[m], bv[m].y, acc[v][1]);
-      acc[v][2] = __builtin_fmaf(ntv[m], bv[m].z, acc[v][2]);
-      acc[v][3] = __builtin_fmaf(ntv[m], bv[m].w, acc[v][3]);
-    }
-  }
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    for (int j = lane + 64 * v + 64 * MIX_PRE; j < ns; j += 256) {
-      const float nt = NT[j];
-      const float4 b = B[j];
-      acc[v][0] = __builtin_fmaf(nt, b.x, acc[v][0]);
-      acc[v][1] = __builtin_fmaf(nt, b.y, acc[v][1]);
-      acc[v][2] = __builtin_fmaf(nt, b.z, acc[v][2]);
-      acc[v][3] = __builtin_fmaf(nt, b.w, acc[v][3]);
-    }
-  }
+  const bool stopped = sim_stopped(d, sim, t);
+  __syncthreads();   // the partials (and the loads above are in flight meanwhile)
+  if (!on) return;
   float part[LP_MAX_STRAINS];
 #pragma unroll
   for (int k = 0; k < LP_MAX_STRAINS; ++k) {
-    float x = (acc[0][k] + acc[2][k]) + (acc[1][k] + acc[3][k]);   // tree levels 128 and 64
-#pragma unroll
-    for (int w = 32; w >= 1; w >>= 1) x = x + __shfl_down(x, w, 64);
-    part[k] = __shfl(x, 0, 64);
+    if (k >= K) { part[k] = 0.0f; continue; }
+    // tree levels 128 and 64, then 32 .. 1 across the wave
+    part[k] = wave_tree_sum_f32((mix[0][w][k][lane] + mix[2][w][k][lane]) + (mix[1][w][k][lane] + mix[3][w][k][lane]));
   }
   if (d.mix_buf) {                 // mix_mode 1: the contraction came from k_mix_mfma
 #pragma unroll
     for (int k = 0; k < LP_MAX_STRAINS; ++k) part[k] = d.mix_buf[(size_t)i * LP_MAX_STRAINS + k];
   }
-  if (off || sim_stopped(d, sim, t)) {
+  if (off || stopped) {
     if (lane == 0) { d.m_round[i] = 0; d.size[i] = 0; d.take_all[i] = 0; }
     return;
   }
@@ -2948,20 +2977,20 @@ __global__ void __launch_bounds__(64) k_mix_mfma(Dev d) {
   }
 }
 
-// Per node: network mix, FOI, count draw.  One wavefront per node.  MINW = 4 keeps at
-// least 4 waves per SIMD (<= 128 VGPRs; one 8-byte value spills, stored at entry and
-// reloaded once), for more nodes than are resident at once, where the network reads need
-// the occupancy; MINW = 1 leaves the kernel unspilled for fewer nodes.
-template <int MINW>
-__global__ void __launch_bounds__(WG, MINW) k_mix_foi(Dev d, int mask) {
+// Per node: network mix, FOI, count draw.  MIX_ROWS nodes per workgroup, one wavefront per
+// node after the mix.
+__global__ void __launch_bounds__(WG) k_mix_foi(Dev d, int mask) {
+  __shared__ float part[WG / 64][MIX_ROWS][LP_MAX_STRAINS][64];
   const int4 dy = today(d);
   const int32_t t = dy.x;
-  const int i = blockIdx.x * (WG / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (i < d.n_nodes) {
-    const int32_t flags = stage_day_flags(dy.y, mask);
-    mix_foi_node(d, i, d.ninfo[i], t, lane, !(flags & LP_DAY_TX));
-  }
+  const int i0 = blockIdx.x * MIX_ROWS;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  if (!d.mix_buf) mix_rows(d, i0, part);
+  const int i = i0 + w;
+  const int32_t flags = stage_day_flags(dy.y, mask);
+  // (wavefronts past the last node take it too, up to the barrier inside)
+  mix_foi_node(d, i < d.n_nodes ? i : d.n_nodes - 1, d.ninfo[i < d.n_nodes ? i : d.n_nodes - 1], t, lane, w,
+               !(flags & LP_DAY_TX), part, i < d.n_nodes);
 }
 
 // One workgroup: plan sampling round `round` (probe offsets over nodes, list space).
