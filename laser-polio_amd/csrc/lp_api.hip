@@ -194,9 +194,8 @@ int32_t host_stage_flags(int32_t flags, int mask) {
   return f;
 }
 
-// Day kind: KIND_RECOUNT, KIND_PLAIN, or the OR of FULL_VD / FULL_RI / FULL_SIA.
-int day_kind(const lp_ctx* c, int32_t t, int mask, int recount) {
-  if (recount) return lp::KIND_RECOUNT;
+// Day kind: KIND_PLAIN, or the OR of FULL_VD / FULL_RI / FULL_SIA.
+int day_kind(const lp_ctx* c, int32_t t, int mask) {
   const int32_t f = host_stage_flags(c->day_flags_h[t], mask);
   return ((f & LP_DAY_VD_STEP) ? lp::FULL_VD : 0) | ((f & LP_DAY_RI) ? lp::FULL_RI : 0) |
          ((f & LP_DAY_SIA) ? lp::FULL_SIA : 0);
@@ -208,8 +207,8 @@ void launch_ei(lp_ctx* c, hipStream_t s, int mask) {
   hipLaunchKernelGGL(lp::k_ei, dim3(c->ei_grid), dim3(lp::WG), 0, s, c->d, mask);
 }
 
-// Agent pass of one day: k_plain over U = tiles per span on plain days,
-// k_full<kind> on FULL days, k_agents in groups of 2 tiles when recounting.
+// Agent pass of one day: k_plain over U = tiles per span on plain days, k_full<kind> on
+// FULL days, the list passes on the list kinds.
 template <int U>
 void launch_agents_u(lp_ctx* c, hipStream_t s, int kind, int mask) {
   const dim3 g(c->n_spans), b(lp::WG);
@@ -223,9 +222,7 @@ void launch_agents_u(lp_ctx* c, hipStream_t s, int kind, int mask) {
     case 5: hipLaunchKernelGGL((lp::k_full<5, true>), g, b, 0, s, c->d, mask); break;
     case 6: hipLaunchKernelGGL((lp::k_full<6, true>), g, b, 0, s, c->d, mask); break;
     case 7: hipLaunchKernelGGL((lp::k_full<7, true>), g, b, 0, s, c->d, mask); break;
-    case lp::KIND_FULL_LIST + 0: case lp::KIND_FULL_LIST + 1: case lp::KIND_FULL_LIST + 2:
-    case lp::KIND_FULL_LIST + 3: case lp::KIND_FULL_LIST + 4: case lp::KIND_FULL_LIST + 5:
-    case lp::KIND_FULL_LIST + 6: {
+    default: {                                            // KIND_FULL_LIST + F - 1
       // DiseaseState from the E / I lists, then births and deaths (only the chunks with a
       // death due or newborn slots), RI from the candidate lists, SIA over the targeted
       // nodes: each stage a pass of its own, in the reference's order, all tallying
@@ -238,16 +235,11 @@ void launch_agents_u(lp_ctx* c, hipStream_t s, int kind, int mask) {
       if (f & lp::FULL_SIA) hipLaunchKernelGGL(lp::k_sia, g, b, 0, s, c->d, mask);
       break;
     }
-    default: hipLaunchKernelGGL((lp::k_agents<2, lp::KIND_RECOUNT>), g, b, 0, s, c->d, mask); break;
   }
 }
 
-// Grid of the record pack / unpack kernels (grid-stride over quads of slots).
-int rec_grid(const lp_ctx* c) {
-  const int64_t nq = (c->cfg.capacity + 3) / 4;
-  const int64_t g = (nq + lp::WG - 1) / lp::WG;
-  return (int)(g < 8192 ? (g > 0 ? g : 1) : 8192);
-}
+// Grid of the passes with one workgroup per tile: span << tpw_sh | tile of the span.
+int tile_grid(const lp_ctx* c) { return c->n_spans << c->d.tpw_sh; }
 
 // Day kinds that process the E / I list; afterwards the records of listed agents
 // keep the timers of when they entered the list until enqueue_actualize.
@@ -266,7 +258,7 @@ void enqueue_actualize(lp_ctx* c) {
 // Bound columns <- device-held state: agent records and actual ri_timer values.
 void enqueue_sync_columns(lp_ctx* c) {
   enqueue_actualize(c);
-  hipLaunchKernelGGL(lp::k_unpack, dim3(rec_grid(c)), dim3(lp::WG), 0, c->stream, c->d);
+  hipLaunchKernelGGL(lp::k_unpack, dim3(tile_grid(c)), dim3(lp::WG), 0, c->stream, c->d);
   hipLaunchKernelGGL(lp::k_ri_sync, dim3(c->n_spans), dim3(lp::WG), 0, c->stream, c->d);
   hipLaunchKernelGGL(lp::k_set_ri_ref, dim3(1), dim3(64), 0, c->stream, c->d, -2);
 }
@@ -285,31 +277,40 @@ void first_run(lp_ctx* c, int32_t t) {
 bool same_list_kind(const lp_ctx* c, int32_t a, int32_t b, int kind) {
   for (int32_t u = a; u < b; ++u) {
     if (!(host_stage_flags(c->day_flags_h[u], LP_STAGE_ALL) & LP_DAY_DS)) return false;
-    int k = day_kind(c, u, LP_STAGE_ALL, 0);
+    int k = day_kind(c, u, LP_STAGE_ALL);
     if (k == lp::KIND_PLAIN) k = lp::KIND_PLAIN_LIST;
-    else if (k >= lp::KIND_FULL && k < lp::KIND_RECOUNT) k = lp::KIND_FULL_LIST + k - lp::KIND_FULL;
+    else if (k >= lp::KIND_FULL && k < lp::KIND_PLAIN_LIST) k = lp::KIND_FULL_LIST + k - lp::KIND_FULL;
     if (k != kind) return false;
   }
   return true;
 }
 
-// The kernel sequence of one tick.  kind: agent-pass variant (KIND_RECOUNT
-// recounts every carried statistic and the paralysis counts); mask: stages;
+// Everything carried from day to day rebuilt from the bound columns, for tick t (the day
+// set by it, `until` as for enqueue_day); with `lists` the E / I list of tick t too; ri: the
+// stages to run include today's RI step.
+void enqueue_recount(lp_ctx* c, int32_t t, int32_t until, bool lists, bool ri) {
+  const int n = std::max(c->cfg.n_nodes, c->n_spans);
+  if (c->rec_dirty) enqueue_sync_columns(c);   // the pass reads the columns
+  hipLaunchKernelGGL(lp::k_recount_begin, dim3(grid_of(n, lp::WG)), dim3(lp::WG), 0, c->stream, c->d, ri ? 1 : 0,
+                     t, until);
+  hipLaunchKernelGGL(lp::k_recount, dim3(tile_grid(c)), dim3(lp::WG), 0, c->stream, c->d, lists ? 1 : 0);
+  c->recount_pending = false;
+  c->rec_dirty = true;
+  c->rec_actual = true;
+}
+
+// The kernel sequence of one tick.  kind: agent-pass variant; mask: stages;
 // tx_adjust: apply today's transmission exposures to the log; advance: move
-// the day counter at the end.
-int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool advance, bool begin) {
-  const int recount = kind == lp::KIND_RECOUNT ? 1 : 0;
+// the day counter at the end; begin: the day begins here, in a call that runs to tick
+// `until` (0: stage calls), not at the end of the day before.
+int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool advance, bool begin, int32_t until = 0) {
   const Dev& d = c->d;
   const int N = c->cfg.n_nodes;
   hipStream_t s = c->stream;
   // passes that read the records need their actual timers (never inside a captured
   // graph: run_days calls enqueue_actualize before capturing)
   if (!list_kind(kind)) enqueue_actualize(c);
-  // a RECOUNT pass reads the bound columns: bring them up to date first; it rebuilds the
-  // RI candidate lists
-  if (recount && c->rec_dirty) enqueue_sync_columns(c);
-  if (recount) HIPCHK(c, hipMemsetAsync(d.ri_lcnt, 0, 2 * (size_t)N * sizeof(int32_t), s));
-  if (begin) hipLaunchKernelGGL(lp::k_day_begin, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask);
+  if (begin) hipLaunchKernelGGL(lp::k_day_begin, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask, t, until);
   const bool ev = c->timing;
   if (ev) {
     if (c->ev_used + 2 > c->ev.size()) {
@@ -328,18 +329,9 @@ int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool ad
     default: launch_agents_u<16>(c, s, kind, mask); break;
   }
   if (ev) { HIPCHK(c, hipEventRecord(c->ev[c->ev_used + 1], s)); c->ev_used += 2; }
-  if (recount) {
-    hipLaunchKernelGGL(lp::k_pack, dim3(rec_grid(c)), dim3(lp::WG), 0, s, d);
-    hipLaunchKernelGGL(lp::k_node_info, dim3(grid_of(N, 256)), dim3(256), 0, s, d);
-    // the pass left ri_timer actual as of today if it ran RI; otherwise it is actual as
-    // of the latest applied RI step, as before the pass
-    const bool ri = host_stage_flags(c->day_flags_h[t], mask) & LP_DAY_RI;
-    hipLaunchKernelGGL(lp::k_set_ri_ref, dim3(1), dim3(64), 0, s, d, ri ? t : -2);
-  }
   // list days tally into node_acc (span partials hold only the carried span weights);
   // the dense passes of the other kinds write every span's partial
-  hipLaunchKernelGGL(lp::k_node_reduce, dim3(N), dim3(lp::WG), 0, s, d, mask, recount,
-                     kind < lp::KIND_PLAIN_LIST ? 0 : 1);
+  hipLaunchKernelGGL(lp::k_node_reduce, dim3(N), dim3(lp::WG), 0, s, d, mask, kind < lp::KIND_PLAIN_LIST ? 0 : 1);
   if (mask & LP_STAGE_TRANSMISSION) {
     if (c->cfg.mix_mode == 1)
       hipLaunchKernelGGL(lp::k_mix_mfma, dim3(c->cfg.n_sims, c->mix_tiles), dim3(64), 0, s, d);
@@ -353,7 +345,9 @@ int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool ad
     else
       hipLaunchKernelGGL((lp::k_finish<512, 6>), dim3(N), dim3(512), 0, s, d);
   }
-  hipLaunchKernelGGL(lp::k_day_end, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask, tx_adjust, advance ? 1 : 0);
+  // (stages before transmission leave it nothing to do)
+  if (advance || (mask & (LP_STAGE_TRANSMISSION | LP_STAGE_LOG)))
+    hipLaunchKernelGGL(lp::k_day_end, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask, tx_adjust, advance ? 1 : 0);
   HIPCHK(c, hipGetLastError());
   c->rec_dirty = true;
   return LP_OK;
@@ -618,30 +612,29 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
   if (t_begin == t_end) return LP_OK;
   first_run(c, t_begin);
   // inside the call each day's k_day_end begins the next day; only the first is begun here
-  hipLaunchKernelGGL(lp::k_set_day, dim3(1), dim3(64), 0, c->stream, c->d, t_begin, t_end);
   bool first = true;
   int rc;
   int32_t t = t_begin;
   if (t == 0) {
-    if ((rc = enqueue_day(c, t, lp::KIND_RECOUNT, LP_STAGE_LOG, 0, true, first))) return rc;
+    // tick 0 only logs; the tally of its dense pass lists the E / I agents for tick 1
+    enqueue_recount(c, t, t_end, false, false);
+    if ((rc = enqueue_day(c, t, lp::KIND_PLAIN, LP_STAGE_LOG, 0, true, first, t_end))) return rc;
     first = false;
-    c->recount_pending = false;
-    c->list_tick = 1;
+    c->list_tick = (c->day_flags_h[0] & LP_DAY_TX) ? 1 : -1;
     t = 1;
   }
   for (; t < t_end; ++t) {
     if (c->recount_pending) {
-      if ((rc = enqueue_day(c, t, lp::KIND_RECOUNT, LP_STAGE_ALL, 1, true, first))) return rc;
-      first = false;
-      c->recount_pending = false;
-      c->list_tick = t + 1;
-      continue;
+      const int32_t f = host_stage_flags(c->day_flags_h[t], LP_STAGE_ALL);
+      const bool lists = f & LP_DAY_DS;
+      enqueue_recount(c, t, t_end, lists, f & LP_DAY_RI);
+      c->list_tick = lists ? t : -1;
     }
-    int kind = day_kind(c, t, LP_STAGE_ALL, 0);
+    int kind = day_kind(c, t, LP_STAGE_ALL);
     // the list kinds keep E / I timers as event days, which needs DiseaseState every day
     if (c->list_tick == t && (host_stage_flags(c->day_flags_h[t], LP_STAGE_ALL) & LP_DAY_DS)) {
       if (kind == lp::KIND_PLAIN) kind = lp::KIND_PLAIN_LIST;
-      else if (kind >= lp::KIND_FULL && kind < lp::KIND_RECOUNT) kind = lp::KIND_FULL_LIST + kind - lp::KIND_FULL;
+      else if (kind >= lp::KIND_FULL && kind < lp::KIND_PLAIN_LIST) kind = lp::KIND_FULL_LIST + kind - lp::KIND_FULL;
     }
     if (list_kind(kind)) c->rec_actual = false;
     else enqueue_actualize(c);
@@ -662,7 +655,7 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
       t += run - 1;
       c->list_tick = t + 1;
     } else {
-      if ((rc = enqueue_day(c, t, kind, LP_STAGE_ALL, 1, true, first))) return rc;
+      if ((rc = enqueue_day(c, t, kind, LP_STAGE_ALL, 1, true, first, t_end))) return rc;
     }
     first = false;
   }
@@ -675,15 +668,11 @@ int lp_step_stage(lp_ctx* c, int32_t t, int32_t mask) {
   if (t < 0 || t >= c->cfg.nt) return fail(c, LP_ERR_ARG, "bad tick");
   if (mask & ~LP_STAGE_ALL) return fail(c, LP_ERR_ARG, "bad stage mask");
   first_run(c, t);
-  hipLaunchKernelGGL(lp::k_set_day, dim3(1), dim3(64), 0, c->stream, c->d, t, 0);
   const bool fused_tx_log = (mask & LP_STAGE_TRANSMISSION) && (mask & LP_STAGE_LOG);
-  const bool log_only = (mask & LP_STAGE_LOG) && !(mask & LP_STAGE_TRANSMISSION);
-  const int recount = (log_only || c->recount_pending) ? 1 : 0;
-  c->recount_pending = false;
   enqueue_actualize(c);
+  if (c->recount_pending) enqueue_recount(c, t, 0, false, host_stage_flags(c->day_flags_h[t], mask) & LP_DAY_RI);
   c->list_tick = -1;   // stage calls do not keep the E / I list
-  return enqueue_day(c, t, day_kind(c, t, mask, recount), mask, fused_tx_log || !(mask & LP_STAGE_LOG) ? 1 : 0, false,
-                     true);
+  return enqueue_day(c, t, day_kind(c, t, mask), mask, fused_tx_log || !(mask & LP_STAGE_LOG) ? 1 : 0, false, true);
 }
 
 int64_t lp_sizeof_init_sim(void) { return (int64_t)sizeof(lp_init_sim); }

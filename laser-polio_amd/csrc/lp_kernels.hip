@@ -11,9 +11,9 @@
 //                  deaths (only chunks with a death due), RI and SIA over the
 //                  node-segmented agent slots, one workgroup per span of tiles;
 //                  k_plain / k_full<F, true> run DiseaseState inline instead when
-//                  no list is available, k_agents when every carried statistic is
-//                  recounted               model.py:1767-1781, 393-454, 1784-1855,
+//                  no list is available        model.py:1767-1781, 393-454, 1784-1855,
 //                                              1994-2060, 980-1007, 902-929
+//                  (k_recount comes before the first day and after host writes)
 //   k_node_reduce  per node: reduce span partials (and k_ei's accumulators), carried
 //                  S / R counts, exclusive prefix of the span weights, result rows
 //                  of VD/DS/RI/SIA
@@ -53,7 +53,7 @@ constexpr int MAX_ROUNDS = 4096;    // bound on the finisher's rounds (each roun
 
 // Tally fields.
 enum : int {
-  P_S = 0, P_SPOS, P_R, P_POTP, P_P, P_DEATHS, P_DPP, P_DP, P_NEWPP, P_NEWP,
+  P_S = 0, P_SPOS, P_R, P_DEATHS = 5, P_DPP, P_DP, P_NEWPP, P_NEWP,
   P_RIV, P_RIP, P_IPV, P_SIAV, P_SIAP,
   P_E0 = 15, P_I0 = 19, P_SIAPK0 = 23, P_SW = 27, P_IB0 = 28
 };
@@ -61,7 +61,7 @@ enum : int {
 enum : int { ERR_CAPACITY = 1, ERR_OVERFLOW = 2, ERR_SAMPLING = 4, ERR_KIND = 8, ERR_LIST = 16 };
 
 // Per-node constants the list and sampling kernels need, gathered in one 64-byte
-// record (rebuilt by k_node_info after every RECOUNT pass).
+// record (rebuilt by every recount).
 struct NodeInfo {
   uint64_t seed, thr_paralysis;
   int64_t slot_base, seg_begin;
@@ -144,7 +144,7 @@ __device__ __forceinline__ bool sim_stopped(const Dev& d, int sim, int t) { retu
 
 // The current day's record at day + 4: {t, day_flags[t], ri_cnt[t], ri_cnt[t + 1]}, so
 // a kernel reads its day, flags and RI counts with one 16-byte load instead of a
-// load that depends on the day counter.  Written where the day is set (k_set_day)
+// load that depends on the day counter.  Written where the day is set (set_day)
 // and where it advances (k_day_end).
 __device__ __forceinline__ int4 today(const Dev& d) { return *reinterpret_cast<const int4*>(d.day + 4); }
 __device__ __forceinline__ int4 day_record(const Dev& d, int32_t t) {
@@ -169,12 +169,12 @@ __device__ __forceinline__ int32_t stage_day_flags(int32_t flags, int mask) {
 }
 
 // ---------------------------------------------------------------------------
-// day[0] = current tick; day[1] = end of the current lp_run_days call (0 outside one).
-__global__ void k_set_day(Dev d, int32_t t, int32_t until) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    set_today(d, day_record(d, t));
-    d.day[1] = until;
-  }
+// day[0] = current tick; day[1] = end of the current lp_run_days call (0 outside one).  Set
+// by the first kernel of a call (k_recount_begin, k_day_begin), which takes both as
+// arguments, so the call needs no launch of its own for it.
+__device__ __forceinline__ void set_day(const Dev& d, int32_t t, int32_t until) {
+  set_today(d, day_record(d, t));
+  d.day[1] = until;
 }
 
 // Kaplan-Meier style age at death (days) for an agent of `age` days, from a
@@ -277,10 +277,12 @@ __device__ void day_stop_check(const Dev& d, int sim, int32_t t, int mask, int c
 
 // Per node: births, per-day resets, early-stop rule.  Inside lp_run_days only the
 // first day launches it: k_day_end of each day begins the next one.
-__global__ void k_day_begin(Dev d, int mask) {
-  const int32_t t = d.day[0];
+__global__ void k_day_begin(Dev d, int mask, int32_t t, int32_t until) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n == 0) d.sel_count[0] = 0;
+  if (n == 0) {
+    set_day(d, t, until);
+    d.sel_count[0] = 0;
+  }
   if (n >= d.n_nodes) return;
   day_begin_node(d, n, t, mask);
   const int sim = d.node_sim[n];
@@ -296,7 +298,7 @@ __global__ void k_day_begin(Dev d, int mask) {
 // wave covers one 256-slot sampling chunk per tile.
 //   phase A  the state words of all U tiles, then the day's campaign / death
 //            columns (dod on VD step days; ri_timer + chronically_missed on RI
-//            days; dob on SIA days; risk only when recounting)
+//            days; dob on SIA days)
 //   phase B  births and deaths                          model.py:1719-1732, 1775-1777
 //   phase C  one vector load per E/I column for every quad holding an E or I agent
 //   phase D  disease progression, RI, SIA and the tallies
@@ -304,9 +306,9 @@ __global__ void k_day_begin(Dev d, int mask) {
 // positive weight, #R; per span and per chunk: the fixed-point weight sum of
 // S agents) are exact integers carried from day to day.  Every change of an
 // agent into or out of S (birth, death, RI, SIA, transmission) or into or out
-// of R applies its exact delta, so only a RECOUNT pass reads every agent's risk.
+// of R applies its exact delta, so only a recount reads every agent's risk.
 // Rare tallies go through LDS atomics; one partial per span, no global atomics.
-enum : int { L_E0 = 0, L_I0 = 4, L_SIAPK0 = 8, L_POTP = 12, L_P, L_DEATHS, L_DPP, L_DP, L_NEWPP, L_NEWP,
+enum : int { L_E0 = 0, L_I0 = 4, L_SIAPK0 = 8, L_DEATHS = 12, L_DPP, L_DP, L_NEWPP, L_NEWP,
              L_RIV, L_RIP, L_IPV, L_SIAV, L_SIAP, L_N };
 
 __device__ __forceinline__ int8_t byte_of(uint32_t w, int a) { return (int8_t)((w >> (8 * a)) & 0xffu); }
@@ -325,13 +327,10 @@ __device__ __forceinline__ void static_for(F&& f) {
 // Day kinds of the agent pass:
 //   PLAIN    no births, deaths, RI or SIA (about 86% of days): k_plain reads the
 //            state column and the E/I columns of quads holding an E or I agent
-//   FULL     VD step / RI / SIA days: k_agents adds the campaign and death columns
-//   RECOUNT  the first pass and any pass after the host changed bound buffers:
-//            k_agents recounts every carried statistic from the agent columns
+//   FULL     VD step / RI / SIA days: births, deaths and the campaigns too
 // FULL days use kinds 1..7 (FULL_* bits); KIND_PLAIN_LIST: a plain day from the E / I list (k_ei);
 // KIND_FULL_LIST + F - 1: FULL day F with DiseaseState from the list (k_ei, then k_full<F, false>)
-enum : int { KIND_PLAIN = 0, KIND_FULL = 1, KIND_RECOUNT = 8, KIND_PLAIN_LIST = 9, KIND_FULL_LIST = 10,
-             N_KINDS = 17 };
+enum : int { KIND_PLAIN = 0, KIND_FULL = 1, KIND_PLAIN_LIST = 8, KIND_FULL_LIST = 9, N_KINDS = 16 };
 
 __device__ __forceinline__ bool is_plain_day(int32_t flags) {
   return !(flags & (LP_DAY_VD_STEP | LP_DAY_RI | LP_DAY_SIA));
@@ -345,12 +344,6 @@ __device__ __forceinline__ bool has_ei_byte(uint32_t w) {
   return ((((x1 - 0x01010101u) & ~x1) | ((x2 - 0x01010101u) & ~x2)) & 0x80808080u) != 0;
 }
 
-// True if any byte of the packed state word equals v (same zero-byte test).
-__device__ __forceinline__ bool has_byte(uint32_t w, uint32_t v) {
-  const uint32_t x = w ^ (v * 0x01010101u);
-  return (((x - 0x01010101u) & ~x) & 0x80808080u) != 0;
-}
-
 // Position of the j-th (0-based) set bit of m; m has more than j set bits.
 __device__ __forceinline__ int nth_set_bit(uint64_t m, int j) {
   int pos = 0;
@@ -362,57 +355,6 @@ __device__ __forceinline__ int nth_set_bit(uint64_t m, int j) {
   return pos;
 }
 
-// Disease progression of one E or I agent (disease_state_step_kernel,
-// model.py:419-452) on the quad's packed columns: a = agent in the quad, s its
-// state (1 or 2, updated), e2 / i2 / p2 the quad's exposure / infection /
-// paralysis timers, ppw its potentially_paralyzed bytes.  Returns true on I -> R.
-__device__ __forceinline__ bool progress_agent(int a, int8_t& s, int strain, uint2& e2, uint2& i2, uint2& p2,
-                                               uint32_t& ppw, uint32_t ipvw, uint64_t seed, uint64_t slot, int32_t t,
-                                               uint64_t thr_paralysis, int8_t* paralyzed_i, int32_t* lc_newpp,
-                                               int32_t* lc_newp) {
-  const int sh16 = 16 * (a & 1);
-  const uint32_t m16 = 0xffffu << sh16;
-  bool to_r = false;
-  if (s == 1) {
-    const uint32_t ew = a < 2 ? e2.x : e2.y;
-    const uint16_t et = (uint16_t)((ew >> sh16) & 0xffffu);
-    if (et == 0) s = 2;
-    else {
-      const uint32_t nw = (ew & ~m16) | ((uint32_t)(et - 1) << sh16);
-      if (a < 2) e2.x = nw; else e2.y = nw;
-    }
-  }
-  if (s == 2) {
-    const uint32_t iw = a < 2 ? i2.x : i2.y;
-    const uint16_t it = (uint16_t)((iw >> sh16) & 0xffffu);
-    if (it == 0) { s = 3; to_r = true; }
-    else {
-      const uint32_t nw = (iw & ~m16) | ((uint32_t)(it - 1) << sh16);
-      if (a < 2) i2.x = nw; else i2.y = nw;
-    }
-    if (strain == 0) {
-      const uint32_t pw = a < 2 ? p2.x : p2.y;
-      const uint16_t pt = (uint16_t)((pw >> sh16) & 0xffffu);
-      if (pt == 0 && byte_of(ppw, a) == -1) {
-        const uint32_t bm = 0xffu << (8 * a);
-        if (byte_of(ipvw, a) == 0) {
-          ppw = (ppw & ~bm) | (1u << (8 * a));
-          atomicAdd(lc_newpp, 1);
-          const uint4 o = draw(seed, slot, t, ST_PARALYSIS);
-          if ((uint64_t)o.x < thr_paralysis) { *paralyzed_i = 1; atomicAdd(lc_newp, 1); }
-        } else {
-          ppw = ppw & ~bm;
-        }
-      }
-      if (pt > 0) {
-        const uint32_t nw = (pw & ~m16) | ((uint32_t)(pt - 1) << sh16);
-        if (a < 2) p2.x = nw; else p2.y = nw;
-      }
-    }
-  }
-  return to_r;
-}
-
 // Agent record (Dev::rec, 16 B per slot): the mutable fields of DiseaseState
 // and the E / I tally in one aligned line segment, so that an E or I agent costs
 // one 16-byte access instead of one cache line from each of seven columns.
@@ -421,7 +363,7 @@ __device__ __forceinline__ bool progress_agent(int a, int8_t& s, int strain, uin
 //   z: daily_infectivity (float bits)
 //   w: ipv_protected (0-7) | paralyzed (8-15) | unused (16-31; the disease state
 //      lives in its column and, for E and I agents, in their list entries)
-// k_pack fills the records from the bound columns after a RECOUNT pass and
+// k_recount fills the records from the bound columns and
 // k_unpack writes them back (lp_sync); in between the records are the state of
 // these fields.  Single fields are written with byte stores (RB_*), so writers
 // of different fields of one record never overwrite each other.
@@ -510,8 +452,8 @@ __global__ void __launch_bounds__(WG) k_ri_sync(Dev d) {
   }
 }
 
-// through >= -1: ri_timer is actual as of tick `through` (after a RECOUNT pass);
-// through < -1: as of the latest applied RI step (after k_ri_sync).
+// through >= -1: ri_timer is actual as of tick `through`; through < -1: as of the latest
+// applied RI step (after k_ri_sync).
 __global__ void k_set_ri_ref(Dev d, int32_t through) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
     const int32_t v = through >= -1 ? through : d.ri_ref[1];
@@ -616,8 +558,8 @@ __device__ __forceinline__ uint4* ei_list_of(const Dev& d, int b, int node) {
   return d.ei_list + (size_t)b * (size_t)d.capacity + d.seg_begin[node];
 }
 
-// Appends one entry (one atomic, returning); for the rare paths (inline DiseaseState,
-// RECOUNT) that append from divergent code.
+// Appends one entry (one atomic, returning); for the rare path (inline DiseaseState)
+// that appends from divergent code.
 __device__ __forceinline__ void append_entry(const Dev& d, int b, int node, const uint4& e) {
   const int pos = atomicAdd(d.ei_cnt + (size_t)b * d.n_nodes + node, 1);
   ei_list_of(d, b, node)[pos] = e;
@@ -740,10 +682,7 @@ __device__ __forceinline__ uint4 exposed_entry(const Dev& d, int64_t slot, int k
   return exposed_entry_rec(slot, d.rec[slot], k, t, rk);
 }
 
-// NodeInfo of every node (one thread per node).
-__global__ void k_node_info(Dev d) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= d.n_nodes) return;
+__device__ __forceinline__ void node_info(const Dev& d, int n) {
   const int sim = d.node_sim[n];
   const lp_sim_params& sp = d.sims[sim];
   NodeInfo ni;
@@ -766,46 +705,189 @@ __global__ void k_node_info(Dev d) {
   d.ninfo[n] = ni;
 }
 
-// Agent records <- bound columns, slots [0, capacity) (one quad per thread).
-__global__ void __launch_bounds__(WG) k_pack(Dev d) {
-  const int64_t nq = (d.capacity + 3) >> 2;
-  for (int64_t q = (int64_t)blockIdx.x * WG + threadIdx.x; q < nq; q += (int64_t)gridDim.x * WG) {
+// ---------------------------------------------------------------------------
+// Recount: everything the library carries from day to day, rebuilt from the bound
+// columns before the first day of a context and before a day that follows a host write
+// of bound buffers (lp_invalidate).  The day itself then runs like any other.
+// k_recount_begin (one thread per node and per span) clears the carried counts, the
+// lists and the span weights and rebuilds the NodeInfo records; ri: today is an RI
+// day the caller runs, so ri_timer is actual as of the tick before it, otherwise as of
+// the latest applied RI step.
+__global__ void __launch_bounds__(WG) k_recount_begin(Dev d, int ri, int32_t t, int32_t until) {
+  const int i = blockIdx.x * WG + threadIdx.x;
+  if (i == 0) {
+    set_day(d, t, until);
+    const int32_t v = ri ? t - 1 : d.ri_ref[1];
+    d.ri_ref[0] = v;
+    d.ri_ref[1] = v;
+  }
+  if (i < d.n_spans) d.partials[(size_t)i * NPART + P_SW] = 0;
+  if (i >= d.n_nodes) return;
+  d.node_carry[(size_t)i * 3 + 0] = 0;
+  d.node_carry[(size_t)i * 3 + 1] = 0;
+  d.node_carry[(size_t)i * 3 + 2] = 0;
+  d.potp_run[i] = 0;
+  d.p_run[i] = 0;
+  d.ei_cnt[(size_t)(t & 1) * d.n_nodes + i] = 0;
+  *ri_cnt_of(d, 0, i) = 0;
+  *ri_cnt_of(d, 1, i) = 0;
+  node_info(d, i);
+}
+
+// One workgroup per tile (blockIdx.x = span << tpw_sh | tile of the span), one quad of slots per
+// thread: the agent records from the columns; per chunk the weight of its S agents and
+// the earliest death date of its live ones; per span its weight; per node #S, #S with
+// positive weight, #R, the potentially paralysed and the paralysed; with `lists` the node's
+// E / I list of today (timers as of the start of today); the RI candidates of the next RI
+// day (today's, if today is one: live agents, not chronically missed, whose window can
+// still open).  Bound by HBM: 28 bytes read and 16 written per slot, every load of a
+// thread in flight at once: 2.45 ms at 269 M slots, 4.8 TB/s, what a large copy reaches.
+// (A pass per span that also ran the day took 2.7 ms there and a separate record pass
+// 3.2 ms; at 5.4 M slots, 330 workgroups of 16 tiles each, 280 and 50 us against 61 us.)
+__global__ void __launch_bounds__(WG) k_recount(Dev d, int lists) {
+  const int4 span = d.spans[blockIdx.x >> d.tpw_sh];
+  const int u = blockIdx.x & ((1 << d.tpw_sh) - 1);
+  if (u >= span.z) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int node = span.x, sim = span.w;
+  const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)tid * 4;
+  const int64_t q0 = i0 >> 2;
+  const int64_t live_hi = d.live_end[node];
+  auto bytes = [&](const void* col) { return reinterpret_cast<const uint32_t*>(col)[q0]; };
+  auto halves = [&](const void* col) { return reinterpret_cast<const uint2*>(col)[q0]; };
+  const uint32_t strain = bytes(d.strain), pp = bytes(d.pp), par = bytes(d.paralyzed), ipv = bytes(d.ipv);
+  const uint2 et = halves(d.exp_timer), it = halves(d.inf_timer), pt = halves(d.par_timer);
+  const float4 inf = reinterpret_cast<const float4*>(d.infect)[q0];
+  const bool any_live = i0 < live_hi;
+  const uint32_t st = any_live ? bytes(d.state) : 0xFFFFFFFFu;
+  const uint32_t missed = any_live ? bytes(d.missed) : 0x01010101u;
+  const uint2 rt = any_live ? halves(d.ri_timer) : make_uint2(0u, 0u);
+  const float4 risk = any_live ? reinterpret_cast<const float4*>(d.risk)[q0] : make_float4(0.f, 0.f, 0.f, 0.f);
+  const int4 dod = any_live ? reinterpret_cast<const int4*>(d.dod)[q0] : make_int4(INT_MAX, INT_MAX, INT_MAX, INT_MAX);
+  const int4 dy = today(d);
+  const int32_t t = dy.x;
+  auto half = [](const uint2& v, int a) { return ((a < 2 ? v.x : v.y) >> (16 * (a & 1))) & 0xffffu; };
+  uint4 rec[4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int64_t i = q * 4 + a;
-      if (i >= d.capacity) break;
-      d.rec[i] = make_uint4((uint32_t)d.exp_timer[i] | ((uint32_t)d.inf_timer[i] << 16),
-                            (uint32_t)d.par_timer[i] | ((uint32_t)(uint8_t)d.strain[i] << 16) |
-                                ((uint32_t)(uint8_t)d.pp[i] << 24),
-                            __float_as_uint(d.infect[i]),
-                            (uint32_t)(uint8_t)d.ipv[i] | ((uint32_t)(uint8_t)d.paralyzed[i] << 8));
+  for (int a = 0; a < 4; ++a) {
+    rec[a] = make_uint4(half(et, a) | (half(it, a) << 16),
+                        half(pt, a) | ((uint32_t)(uint8_t)byte_of(strain, a) << 16) | ((uint32_t)(uint8_t)byte_of(pp, a) << 24),
+                        __float_as_uint(lane_of(inf, a)),
+                        (uint32_t)(uint8_t)byte_of(ipv, a) | ((uint32_t)(uint8_t)byte_of(par, a) << 8));
+    d.rec[i0 + a] = rec[a];
+  }
+  if (d.stop_day[sim] < t) return;                        // stopped: nothing of it is carried any more (uniform)
+  const int32_t step = d.sims[sim].ri_step;
+  int32_t dmin = INT_MAX;
+  int64_t cw = 0;
+  uint32_t c_n = 0, c_p = 0, ei = 0, cand = 0;             // counts of 10 bits: S, S weighing, R; paralysed ones
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int8_t s = byte_of(st, a);
+    if (i0 + a >= live_hi || s < 0) continue;
+    const int32_t dd = lane_of(dod, a);
+    dmin = dd < dmin ? dd : dmin;
+    if (s == 0) {
+      const int64_t w = weight_q24(lane_of(risk, a));
+      cw += w;
+      c_n += 1u + (w > 0 ? 1u << 10 : 0u);
+    } else if (s == 3) {
+      c_n += 1u << 20;
+    } else if (s == 1 || s == 2) {
+      ei |= 1u << a;
     }
+    c_p += (byte_of(pp, a) == 1 ? 1u : 0u) + (byte_of(par, a) == 1 ? 1u << 16 : 0u);
+    if (byte_of(missed, a) != 1 && (int16_t)half(rt, a) > -step) cand |= 1u << a;
+  }
+  const int64_t c = (i0 >> 8);
+  cw = wave_sum_i64(cw);
+  dmin = wave_min_i32(dmin);
+  c_n = (uint32_t)wave_sum_i32((int32_t)c_n);             // at most 256 each
+  if (__ballot(c_p != 0)) c_p = (uint32_t)wave_sum_i32((int32_t)c_p);
+  if (lane == 0) { d.chunk_sum[c] = cw; d.chunk_min_dod[c] = dmin; }
+  // the tile's counts, weight and list reservations: one atomic per field and workgroup (a
+  // wavefront's own atomics on one node's list lengths serialised: 214 us for 5.4 M slots
+  // of 14 nodes whose every agent was an RI candidate).  Without an RI day ahead no
+  // candidates are listed.
+  const bool ri_ahead = d.ri_cnt[d.nt] > dy.z;
+  if (!lists) ei = 0;
+  if (!ri_ahead) cand = 0;
+  const int32_t mine = __popc(ei) | (__popc(cand) << 16);  // at most 256 of each in a wave
+  const int32_t incl = wave_incl_scan_i32(mine);
+  __shared__ int64_t s_w[WG / 64];
+  __shared__ uint32_t s_n[WG / 64], s_p[WG / 64];
+  __shared__ int32_t s_l[WG / 64], s_base[2];
+  if (lane == 63) { s_w[wave] = cw; s_n[wave] = c_n; s_p[wave] = c_p; s_l[wave] = incl; }
+  __syncthreads();
+  const int b = dy.z & 1;
+  if (tid < 8) {
+    int64_t v = 0;
+#pragma unroll
+    for (int w = 0; w < WG / 64; ++w)
+      v += tid == 0 ? s_w[w] : tid < 4 ? (int64_t)((s_n[w] >> (10 * (tid - 1))) & 0x3ffu)
+         : tid < 6 ? (int64_t)((s_p[w] >> (16 * (tid - 4))) & 0xffffu) : (int64_t)((s_l[w] >> (16 * (tid - 6))) & 0xffff);
+    if (v != 0) {
+      if (tid == 0)
+        atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(blockIdx.x >> d.tpw_sh) * NPART + P_SW),
+                  (unsigned long long)v);
+      else if (tid < 4)
+        atomicAdd(reinterpret_cast<unsigned long long*>(d.node_carry + (size_t)node * 3 + tid - 1), (unsigned long long)v);
+      else if (tid < 6)
+        atomicAdd((tid == 4 ? d.potp_run : d.p_run) + node, (int32_t)v);
+      else
+        s_base[tid - 6] = atomicAdd(tid == 6 ? d.ei_cnt + (size_t)(t & 1) * d.n_nodes + node : ri_cnt_of(d, b, node),
+                                    (int32_t)v);
+    }
+  }
+  __syncthreads();
+  int before = incl - mine;
+  for (int w = 0; w < wave; ++w) before += s_l[w];
+  if (ei) {
+    uint4* L = ei_list_of(d, t & 1, node) + s_base[0] + (before & 0xffff);
+    const float* r0k = d.sims[sim].strain_r0;
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      if ((ei >> a) & 1u) *L++ = entry_from_rec((uint32_t)(i0 + a), byte_of(st, a), rec[a], t, r0k);
+  }
+  if (cand) {
+    uint32_t* L = ri_list_of(d, b, node) + s_base[1] + (before >> 16);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+      if ((cand >> a) & 1u) *L++ = (uint32_t)(i0 + a);
   }
 }
 
-// Bound columns <- agent records (daily_infectivity is never written, so not copied back).
+// Bound columns <- agent records, one workgroup per tile as k_recount, one quad per thread
+// (daily_infectivity is never written, so not copied back; nor is a slot no agent has
+// held yet).  Bound by HBM: 27 bytes a live slot in 16-, 8- and 4-byte accesses, 1.25 ms
+// for 227 M agents in 269 M slots (4.9 TB/s; byte stores over every slot took 2.6 ms).
 __global__ void __launch_bounds__(WG) k_unpack(Dev d) {
-  const int64_t nq = (d.capacity + 3) >> 2;
-  for (int64_t q = (int64_t)blockIdx.x * WG + threadIdx.x; q < nq; q += (int64_t)gridDim.x * WG) {
+  const int4 span = d.spans[blockIdx.x >> d.tpw_sh];
+  const int u = blockIdx.x & ((1 << d.tpw_sh) - 1);
+  const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)threadIdx.x * 4;
+  if (u >= span.z || i0 >= d.live_end[span.x]) return;
+  const int64_t q0 = i0 >> 2;
+  uint4 r[4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int64_t i = q * 4 + a;
-      if (i >= d.capacity) break;
-      const uint4 r = d.rec[i];
-      d.exp_timer[i] = (uint16_t)(r.x & 0xffffu);
-      d.inf_timer[i] = (uint16_t)(r.x >> 16);
-      d.par_timer[i] = (uint16_t)(r.y & 0xffffu);
-      d.strain[i] = (int8_t)(r.y >> 16);
-      d.pp[i] = (int8_t)(r.y >> 24);
-      d.ipv[i] = (int8_t)(r.w & 0xffu);
-      d.paralyzed[i] = (int8_t)(r.w >> 8);
-    }
-  }
+  for (int a = 0; a < 4; ++a) r[a] = d.rec[i0 + a];
+  auto halves = [](uint32_t a, uint32_t b, uint32_t c, uint32_t e) {
+    return make_uint2((a & 0xffffu) | (b << 16), (c & 0xffffu) | (e << 16));
+  };
+  auto bytes = [](uint32_t a, uint32_t b, uint32_t c, uint32_t e) {
+    return (a & 0xffu) | ((b & 0xffu) << 8) | ((c & 0xffu) << 16) | (e << 24);
+  };
+  reinterpret_cast<uint2*>(d.exp_timer)[q0] = halves(r[0].x, r[1].x, r[2].x, r[3].x);
+  reinterpret_cast<uint2*>(d.inf_timer)[q0] = halves(r[0].x >> 16, r[1].x >> 16, r[2].x >> 16, r[3].x >> 16);
+  reinterpret_cast<uint2*>(d.par_timer)[q0] = halves(r[0].y, r[1].y, r[2].y, r[3].y);
+  reinterpret_cast<uint32_t*>(d.strain)[q0] = bytes(r[0].y >> 16, r[1].y >> 16, r[2].y >> 16, r[3].y >> 16);
+  reinterpret_cast<uint32_t*>(d.pp)[q0] = bytes(r[0].y >> 24, r[1].y >> 24, r[2].y >> 24, r[3].y >> 24);
+  reinterpret_cast<uint32_t*>(d.ipv)[q0] = bytes(r[0].w, r[1].w, r[2].w, r[3].w);
+  reinterpret_cast<uint32_t*>(d.paralyzed)[q0] = bytes(r[0].w >> 8, r[1].w >> 8, r[2].w >> 8, r[3].w >> 8);
 }
 
 // Writes the span partial: carried-count deltas from red[][], tallies from LDS.
 __device__ __forceinline__ void write_partial(const Dev& d, int tid, const int64_t (*red)[4], const int32_t* lc,
-                                              const unsigned long long* lib, bool recount, bool sw_delta) {
+                                              const unsigned long long* lib, bool sw_delta) {
   if (tid >= NPART) return;
   int64_t v = 0;
   if (tid == P_S || tid == P_SPOS || tid == P_R || tid == P_SW) {
@@ -818,8 +900,6 @@ __device__ __forceinline__ void write_partial(const Dev& d, int tid, const int64
   else if (tid >= P_IB0 && tid < P_IB0 + 4) v = (int64_t)lib[tid - P_IB0];
   else {
     switch (tid) {
-      case P_POTP: v = lc[L_POTP]; break;
-      case P_P: v = lc[L_P]; break;
       case P_DEATHS: v = lc[L_DEATHS]; break;
       case P_DPP: v = lc[L_DPP]; break;
       case P_DP: v = lc[L_DP]; break;
@@ -835,7 +915,6 @@ __device__ __forceinline__ void write_partial(const Dev& d, int tid, const int64
   }
   int64_t* slot = d.partials + (size_t)blockIdx.x * NPART + tid;
   if (tid != P_SW) *slot = v;
-  else if (recount) *slot = v;
   else if (sw_delta && v != 0)   // the carried weight: a delta, added without a dependent load
     atomicAdd(reinterpret_cast<unsigned long long*>(slot), (unsigned long long)v);
 }
@@ -848,6 +927,11 @@ __device__ __forceinline__ void write_partial(const Dev& d, int tid, const int64
 // S statistics do not change on these days; I -> R adds to the R delta.
 template <int U>
 __global__ void __launch_bounds__(WG) k_plain(Dev d, int mask) {
+  if (!(mask & (LP_STAGE_DISEASE | LP_STAGE_TRANSMISSION | LP_STAGE_LOG))) {
+    // a stage call with nothing to do on this day: no agent is read
+    if (threadIdx.x < NPART && threadIdx.x != P_SW) d.partials[(size_t)blockIdx.x * NPART + threadIdx.x] = 0;
+    return;
+  }
   const int4 span = d.spans[blockIdx.x];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   __shared__ uint32_t s_st[U][WG];
@@ -915,7 +999,7 @@ __global__ void __launch_bounds__(WG) k_plain(Dev d, int mask) {
     if (lane == 0) { red[wave][0] = 0; red[wave][1] = 0; red[wave][2] = a2; red[wave][3] = 0; }
   }
   __syncthreads();
-  write_partial(d, tid, red, lc, lib, false, false);
+  write_partial(d, tid, red, lc, lib, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -1699,7 +1783,7 @@ __global__ void __launch_bounds__(WG, 5) k_full(Dev d, int mask) {
     if (lane == 0) { red[wave][0] = a0; red[wave][1] = a1; red[wave][2] = a2; red[wave][3] = a3; }
   }
   __syncthreads();
-  write_partial(d, tid, red, lc, lib, false, true);
+  write_partial(d, tid, red, lc, lib, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -2113,351 +2197,6 @@ __global__ void __launch_bounds__(WG) k_sia(Dev d, int mask) {
 }
 
 // ---------------------------------------------------------------------------
-// RECOUNT passes: the span's tiles in groups of G, each group through phases
-// A-D (every agent's risk, paralysis flags and state recounted); tallies
-// accumulate over the groups, one partial per span.
-template <int G, int KIND>
-__global__ void __launch_bounds__(WG) k_agents(Dev d, int mask) {
-  constexpr bool RECOUNT = KIND == KIND_RECOUNT;
-  const int4 span0 = d.spans[blockIdx.x];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int4 dy = today(d);
-  const int32_t t = dy.x;
-  const int node = span0.x, sim = span0.w;
-  const int64_t live_hi = d.live_end[node];
-  const int32_t stop_day = d.stop_day[sim];
-  const int32_t flags = stage_day_flags(dy.y, mask);
-  if (stop_day < t) return;
-  if (!RECOUNT && is_plain_day(flags)) {
-    if (tid < NPART && tid != P_SW) d.partials[(size_t)blockIdx.x * NPART + tid] = 0;
-    if (tid == 0) atomicOr(d.err, ERR_KIND);
-    return;
-  }
-  const bool do_deaths = flags & LP_DAY_VD_STEP;
-  const bool do_ds = flags & LP_DAY_DS;
-  const bool do_ri = flags & LP_DAY_RI;
-  const bool do_sia = flags & LP_DAY_SIA;
-  const bool do_tally = (flags & LP_DAY_TX) != 0;
-  const bool need_ei = do_ds || do_tally;
-  const int32_t sia_b = do_sia ? d.day_sia_begin[t] : 0;
-  const int32_t sia_n = do_sia ? d.day_sia_count[t] : 0;
-
-  __shared__ int32_t lc[L_N];
-  __shared__ unsigned long long lib[LP_MAX_STRAINS];
-  __shared__ int64_t red[WG / 64][4];
-
-  const lp_sim_params& sp = d.sims[sim];
-  const int64_t nb_lo = d.nb_begin[node];
-  const uint64_t seed = sp.seed;
-  const int64_t sbase = sp.slot_base;
-  const uint64_t thr_ri = do_ri ? d.thr_ri[node] : 0, thr_ipv = do_ri ? d.thr_ipv[node] : 0;
-  if (tid < L_N) lc[tid] = 0;
-  if (tid < LP_MAX_STRAINS) lib[tid] = 0;
-  __syncthreads();
-
-  // carried-statistic deltas (absolute counts when recounting)
-  int32_t c_s = 0, c_spos = 0, c_r = 0;
-  int64_t c_sw = 0;
-
-  for (int g0 = 0; g0 < span0.z; g0 += G) {
-    const int4 span = make_int4(node, span0.y + g0, span0.z - g0 < G ? span0.z - g0 : G, sim);
-    // ---- phase A ----
-    uint32_t st[G], st0[G];
-    float4 rk[G];
-    int4 dd[G], db[G];
-    uint2 rt[G];
-    uint32_t mw[G];
-    bool tv[G];
-    static_for<G>([&](auto uc) {
-      constexpr int u = decltype(uc)::value;
-      const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)tid * 4;
-      const bool v = (u < span.z) && (i0 < live_hi);
-      tv[u] = v;
-      st[u] = (u < span.z) ? reinterpret_cast<const uint32_t*>(d.state)[i0 >> 2] : 0xFFFFFFFFu;
-      st0[u] = st[u];
-      if (RECOUNT) rk[u] = v ? *reinterpret_cast<const float4*>(d.risk + i0) : make_float4(0.f, 0.f, 0.f, 0.f);
-      if (do_deaths || RECOUNT) dd[u] = v ? *reinterpret_cast<const int4*>(d.dod + i0) : make_int4(INT_MAX, INT_MAX, INT_MAX, INT_MAX);
-      if (do_ri || do_sia) mw[u] = v ? reinterpret_cast<const uint32_t*>(d.missed)[i0 >> 2] : 0x01010101u;
-      if (do_ri) rt[u] = v ? *reinterpret_cast<const uint2*>(d.ri_timer + i0) : make_uint2(0u, 0u);
-      if (do_sia) db[u] = v ? *reinterpret_cast<const int4*>(d.dob + i0) : make_int4(0, 0, 0, 0);
-    });
-    int64_t cw[G];
-    static_for<G>([&](auto uc) { cw[decltype(uc)::value] = 0; });
-
-    // ---- phase B: births and deaths ----
-    const bool vd_work = do_deaths || nb_lo < live_hi;
-    bool ei[G];
-    static_for<G>([&](auto uc) {
-      constexpr int u = decltype(uc)::value;
-      const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)tid * 4;
-      bool any = false;
-      if (tv[u]) {
-        if (vd_work) {
-#pragma unroll
-          for (int a = 0; a < 4; ++a) {
-            const int64_t i = i0 + a;
-            if (i >= live_hi) continue;
-            int8_t s = byte_of(st[u], a);
-            if (i >= nb_lo) {
-              const uint64_t slot = (uint64_t)(i - sbase);
-              d.dob[i] = t;
-              d.dod[i] = t + km_age_at_death(d.km_cd + (size_t)sim * LP_KM_LEN, seed, slot, t, 0);
-              d.node_id[i] = (int16_t)(node - sp.node_begin);   // sim-local node id
-              if (sp.newborn_ri_timer >= 0) {
-                d.ri_timer[i] = (int16_t)sp.newborn_ri_timer;
-                if (do_ri) {
-                  const uint32_t hv = (uint32_t)(uint16_t)sp.newborn_ri_timer << (16 * (a & 1));
-                  const uint32_t hm = 0xffffu << (16 * (a & 1));
-                  if (a < 2) rt[u].x = (rt[u].x & ~hm) | hv; else rt[u].y = (rt[u].y & ~hm) | hv;
-                }
-              }
-              if (do_sia) { if (a == 0) db[u].x = t; else if (a == 1) db[u].y = t; else if (a == 2) db[u].z = t; else db[u].w = t; }
-              if (!RECOUNT) {                             // a newborn enters S
-                const int64_t w = weight_q24(d.risk[i]);
-                c_s += 1; c_spos += (w > 0); c_sw += w; cw[u] += w;
-              }
-              s = 0;
-            } else if (do_deaths && s >= 0 && lane_of(dd[u], a) <= t) {
-              atomicAdd(&lc[L_DEATHS], 1);
-              if (d.pp[i] == 1) atomicAdd(&lc[L_DPP], 1);
-              if (d.paralyzed[i] == 1) atomicAdd(&lc[L_DP], 1);
-              if (!RECOUNT) {
-                if (s == 0) {                             // a susceptible leaves S
-                  const int64_t w = weight_q24(d.risk[i]);
-                  c_s -= 1; c_spos -= (w > 0); c_sw -= w; cw[u] -= w;
-                } else if (s == 3) {
-                  c_r -= 1;
-                }
-              }
-              s = -1;
-            }
-            st[u] = (st[u] & ~(0xffu << (8 * a))) | ((uint32_t)(uint8_t)s << (8 * a));
-          }
-        }
-        const uint32_t w = st[u];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const int8_t s = byte_of(w, a);
-          any = any || ((s == 1 || s == 2) && i0 + a < live_hi);
-        }
-      }
-      ei[u] = any && need_ei;
-    });
-    if (RECOUNT) {
-      // earliest death date among each chunk's live agents (date_of_death of newborns just written)
-      static_for<G>([&](auto uc) {
-        constexpr int u = decltype(uc)::value;
-        const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)tid * 4;
-        int32_t dmin = INT_MAX;
-        if (tv[u]) {
-#pragma unroll
-          for (int a = 0; a < 4; ++a) {
-            const int64_t i = i0 + a;
-            if (i >= live_hi || byte_of(st[u], a) < 0) continue;
-            const int32_t dod = i >= nb_lo ? d.dod[i] : lane_of(dd[u], a);
-            dmin = dod < dmin ? dod : dmin;
-          }
-        }
-        if (u < span.z) {
-          const int32_t wm = wave_min_i32(dmin);
-          if (lane == 0) d.chunk_min_dod[((int64_t)span.y + u) * (LP_TILE / LP_CHUNK) + wave] = wm;
-        }
-      });
-    }
-
-    // ---- phase C: E/I columns of quads holding an E or I agent ----
-    uint2 xe[G], xi[G], xp[G];
-    uint32_t xs[G], xpp[G], xipv[G];
-    float4 xin[G];
-    static_for<G>([&](auto uc) {
-      constexpr int u = decltype(uc)::value;
-      const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)tid * 4;
-      if (ei[u]) {
-        xe[u] = *reinterpret_cast<const uint2*>(d.exp_timer + i0);
-        xi[u] = *reinterpret_cast<const uint2*>(d.inf_timer + i0);
-        xp[u] = *reinterpret_cast<const uint2*>(d.par_timer + i0);
-        xs[u] = reinterpret_cast<const uint32_t*>(d.strain)[i0 >> 2];
-        xpp[u] = reinterpret_cast<const uint32_t*>(d.pp)[i0 >> 2];
-        xipv[u] = reinterpret_cast<const uint32_t*>(d.ipv)[i0 >> 2];
-        xin[u] = do_tally ? *reinterpret_cast<const float4*>(d.infect + i0) : make_float4(0.f, 0.f, 0.f, 0.f);
-      } else {
-        xe[u] = xi[u] = xp[u] = make_uint2(0u, 0u);
-        xs[u] = xpp[u] = xipv[u] = 0u;
-        xin[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      }
-    });
-
-    // ---- phase D: progression, RI, SIA, tallies ----
-    static_for<G>([&](auto uc) {
-      constexpr int u = decltype(uc)::value;
-      const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)tid * 4;
-      uint32_t wf = st[u];   // the quad's state word after the pass
-      if (tv[u] && !ei[u] && !do_ri && !do_sia) {
-        // no E/I in the quad and no campaign today: only a recount looks at it
-        if (RECOUNT) {
-#pragma unroll
-          for (int a = 0; a < 4; ++a) {
-            const int8_t s = byte_of(st[u], a);
-            const bool live = i0 + a < live_hi;
-            if (live && s == 0) {
-              const int64_t wt = weight_q24(lane_of(rk[u], a));
-              c_s += 1; c_spos += (wt > 0); c_sw += wt; cw[u] += wt;
-            }
-            c_r += (live && s == 3);
-            if (live && s >= 0 && d.paralyzed[i0 + a] == 1) atomicAdd(&lc[L_P], 1);
-            if (live && s >= 0 && d.pp[i0 + a] == 1) atomicAdd(&lc[L_POTP], 1);
-          }
-        }
-        if (vd_work && st[u] != st0[u]) reinterpret_cast<uint32_t*>(d.state)[i0 >> 2] = st[u];
-      } else if (tv[u]) {
-        uint32_t w = st[u];
-        uint2 e2 = xe[u], i2 = xi[u], p2 = xp[u], r2 = do_ri ? rt[u] : make_uint2(0u, 0u);
-        uint32_t ppw = xpp[u];
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const int64_t i = i0 + a;
-          if (i >= live_hi) continue;
-          int8_t s = byte_of(w, a);
-          const uint64_t slot = (uint64_t)(i - sbase);
-          int k = byte_of(xs[u], a) & (LP_MAX_STRAINS - 1);
-          const int sh16 = 16 * (a & 1);
-          const uint32_t m16 = 0xffffu << sh16;
-          if (do_ds && (s == 1 || s == 2)) {
-            if (progress_agent(a, s, byte_of(xs[u], a), e2, i2, p2, ppw, xipv[u], seed, slot, t, sp.thr_paralysis,
-                               d.paralyzed + i, &lc[L_NEWPP], &lc[L_NEWP]) && !RECOUNT)
-              c_r += 1;                                   // I -> R
-          }
-          if ((do_ri || do_sia) && s >= 0 && byte_of(mw[u], a) != 1) {
-            const int8_t s_before = s;
-            if (do_ri) {                                  // fast_ri (model.py:1826-1854)
-              const int32_t step = sp.ri_step;
-              const uint32_t rw = a < 2 ? r2.x : r2.y;
-              const int16_t timer = (int16_t)((int16_t)((rw >> sh16) & 0xffffu) - step);
-              const uint32_t nw = (rw & ~m16) | ((uint32_t)(uint16_t)timer << sh16);
-              if (a < 2) r2.x = nw; else r2.y = nw;
-              bool eligible = false;
-              if (t == step) eligible = timer <= 0 && timer >= -step;
-              else if (t > step) eligible = timer <= 0 && timer > -step;
-              if (eligible) {
-                const uint4 o = draw(seed, slot, t, ST_RI);
-                if ((uint64_t)o.x < thr_ri) {
-                  atomicAdd(&lc[L_RIV], 1);
-                  if (s == 0) { s = 1; k = sp.ri_strain; d.strain[i] = (int8_t)k; atomicAdd(&lc[L_RIP], 1); }
-                }
-                if ((uint64_t)o.y < thr_ipv) { atomicAdd(&lc[L_IPV], 1); d.ipv[i] = 1; }
-              }
-            }
-            if (do_sia) {                                 // fast_sia (model.py:2033-2059), per event
-              const int32_t age = t - lane_of(db[u], a);
-              for (int e = 0; e < sia_n; ++e) {
-                const int ev = sia_b + e;
-                if (!(d.sia_min_age[ev] <= age && age <= d.sia_max_age[ev])) continue;
-                const uint64_t t1 = d.sia_thr[((size_t)ev * d.n_nodes + node) * 2];
-                if (t1 == 0) continue;
-                const uint4 o = draw(seed, slot, t, ST_SIA | ((uint32_t)e << 8));
-                if ((uint64_t)o.x < t1) {
-                  const bool last = (e == sia_n - 1);
-                  if (last) atomicAdd(&lc[L_SIAV], 1);
-                  if (s == 0 && (uint64_t)o.x < d.sia_thr[((size_t)ev * d.n_nodes + node) * 2 + 1]) {
-                    s = 1;
-                    k = d.sia_strain[ev] & (LP_MAX_STRAINS - 1);
-                    d.strain[i] = (int8_t)k;
-                    atomicAdd(&lc[L_SIAPK0 + k], 1);
-                    if (last) atomicAdd(&lc[L_SIAP], 1);
-                  }
-                }
-              }
-            }
-            if (!RECOUNT && s_before == 0 && s != 0) {    // vaccinated out of S
-              const int64_t wt = weight_q24(d.risk[i]);
-              c_s -= 1; c_spos -= (wt > 0); c_sw -= wt; cw[u] -= wt;
-            }
-          }
-          if (s >= 0) {
-            if (RECOUNT) {
-              if (s == 0) {
-                const int64_t wt = weight_q24(lane_of(rk[u], a));
-                c_s += 1; c_spos += (wt > 0); c_sw += wt; cw[u] += wt;
-              } else if (s == 3) {
-                c_r += 1;
-              }
-              if (d.pp[i] == 1 || byte_of(ppw, a) == 1) atomicAdd(&lc[L_POTP], 1);
-              if (d.paralyzed[i] == 1) atomicAdd(&lc[L_P], 1);
-            }
-            if (do_tally) {                               // tx_step_prep / count_SEIRP tally of E and I
-              if (s == 1) {
-                atomicAdd(&lc[L_E0 + k], 1);
-              } else if (s == 2) {
-                atomicAdd(&lc[L_I0 + k], 1);
-                const int64_t wv = weight_q24(lane_of(xin[u], a) * sp.strain_r0[k]);
-                atomicAdd(&lib[k], (unsigned long long)wv);
-              }
-            }
-          }
-          w = (w & ~(0xffu << (8 * a))) | ((uint32_t)(uint8_t)s << (8 * a));
-        }
-        if (w != st0[u]) reinterpret_cast<uint32_t*>(d.state)[i0 >> 2] = w;
-        wf = w;
-        if (ei[u]) {
-          if (e2.x != xe[u].x || e2.y != xe[u].y) *reinterpret_cast<uint2*>(d.exp_timer + i0) = e2;
-          if (i2.x != xi[u].x || i2.y != xi[u].y) *reinterpret_cast<uint2*>(d.inf_timer + i0) = i2;
-          if (p2.x != xp[u].x || p2.y != xp[u].y) *reinterpret_cast<uint2*>(d.par_timer + i0) = p2;
-          if (ppw != xpp[u]) reinterpret_cast<uint32_t*>(d.pp)[i0 >> 2] = ppw;
-        }
-        if (do_ri && (r2.x != rt[u].x || r2.y != rt[u].y)) *reinterpret_cast<uint2*>(d.ri_timer + i0) = r2;
-      }
-      if (u < span.z) {                                   // E / I list of the next day (uniform condition)
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const int8_t s = byte_of(wf, a);
-          if (!(tv[u] && i0 + a < live_hi && (s == 1 || s == 2))) continue;
-          const int64_t i = i0 + a;   // timers as written by this pass: as of tomorrow
-          const int k = d.strain[i] & (LP_MAX_STRAINS - 1);
-          const int64_t w = weight_q24(d.infect[i] * sp.strain_r0[k]);
-          const uint4 e = s == 1 ? entry_e((uint32_t)i, k, d.exp_timer[i], d.inf_timer[i], d.par_timer[i], d.pp[i],
-                                           t + 1, w)
-                                 : entry_i((uint32_t)i, k, d.inf_timer[i], d.par_timer[i], d.pp[i], t + 1, w);
-          append_entry(d, (t + 1) & 1, node, e);
-        }
-        // RI candidates: live agents not chronically missed whose window can still open
-        // (ri_timer is actual here; re-read after this pass's own RI step)
-        uint32_t rb = 0;
-        if (tv[u]) {
-          const uint2 rr = *reinterpret_cast<const uint2*>(d.ri_timer + i0);
-          const uint32_t mm = reinterpret_cast<const uint32_t*>(d.missed)[i0 >> 2];
-#pragma unroll
-          for (int a = 0; a < 4; ++a) {
-            const int16_t tm = (int16_t)(((a < 2 ? rr.x : rr.y) >> (16 * (a & 1))) & 0xffffu);
-            if (i0 + a < live_hi && byte_of(wf, a) >= 0 && byte_of(mm, a) != 1 && tm > -sp.ri_step) rb |= 1u << a;
-          }
-        }
-        const int rbuf = dy.w & 1;
-        wave_append_quad_to(ri_list_of(d, rbuf, node), ri_cnt_of(d, rbuf, node), i0, rb, lane);
-      }
-      // chunk weight sums: rewritten when recounting, adjusted by their delta otherwise
-      // (the condition is uniform over the workgroup: wave_sum needs every lane)
-      if (u < span.z && (RECOUNT || ((int64_t)span.y + u) * LP_TILE < live_hi)) {
-        const int64_t cs = wave_sum_i64(cw[u]);
-        const int64_t c = (((int64_t)span.y + u) * LP_TILE >> 8) + wave;
-        if (lane == 0) {
-          if (RECOUNT) d.chunk_sum[c] = cs;
-          else if (cs != 0) d.chunk_sum[c] += cs;
-        }
-      }
-    });
-  }
-
-  // ---- span partial ----
-  {
-    const int32_t a0 = wave_sum_i32(c_s), a1 = wave_sum_i32(c_spos), a2 = wave_sum_i32(c_r);
-    const int64_t a3 = wave_sum_i64(c_sw);
-    if (lane == 0) { red[wave][0] = a0; red[wave][1] = a1; red[wave][2] = a2; red[wave][3] = a3; }
-  }
-  __syncthreads();
-  write_partial(d, tid, red, lc, lib, RECOUNT, true);
-}
-
-// ---------------------------------------------------------------------------
 // Exclusive scan of a node's span weights (partial field P_SW of spans [s0, s1))
 // into prefix[s]; returns the total.  One wavefront scans 64 spans per step.
 // ATOMIC_IO reads the weights / writes the prefix with agent-scope atomics.
@@ -2491,7 +2230,7 @@ __device__ int64_t node_span_scan(int64_t* partials, int64_t* prefix, int s0, in
 }
 
 // Per node: reduce span partials, span prefix, results rows of VD / DS / RI / SIA.
-__global__ void __launch_bounds__(WG) k_node_reduce(Dev d, int mask, int recount, int list) {
+__global__ void __launch_bounds__(WG) k_node_reduce(Dev d, int mask, int list) {
   const int4 dy = today(d);
   const int32_t t = dy.x;
   const int n = blockIdx.x;
@@ -2573,7 +2312,7 @@ __global__ void __launch_bounds__(WG) k_node_reduce(Dev d, int mask, int recount
   if (tid < 3) {
     // carried per-node counts: S, S with positive weight, R (the spans hold deltas)
     const int f = tid == 0 ? P_S : tid == 1 ? P_SPOS : P_R;
-    const int64_t v = recount ? tally[f] : carry0 + tally[f];
+    const int64_t v = carry0 + tally[f];
     d.node_carry[(size_t)n * 3 + tid] = v;
     tally[f] = v;
   }
@@ -2632,13 +2371,8 @@ __global__ void __launch_bounds__(WG) k_node_reduce(Dev d, int mask, int recount
     }
     d.r_newexp[row + n] += tot;
   }
-  if (recount) {
-    d.potp_run[n] = (int32_t)tally[P_POTP];
-    d.p_run[n] = (int32_t)tally[P_P];
-  } else {
-    d.potp_run[n] += (int32_t)(tally[P_NEWPP] - tally[P_DPP]);
-    d.p_run[n] += (int32_t)(tally[P_NEWP] - tally[P_DP]);
-  }
+  d.potp_run[n] += (int32_t)(tally[P_NEWPP] - tally[P_DPP]);
+  d.p_run[n] += (int32_t)(tally[P_NEWP] - tally[P_DP]);
 }
 
 // ---------------------------------------------------------------------------
