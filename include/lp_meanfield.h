@@ -14,6 +14,11 @@
  * only); these entry points exist for gradient-based calibration of r0_scalars,
  * the gravity parameters and seasonality against ABM output.
  *
+ * Up to 256 nodes one workgroup rolls all days of a call; up to 2048 nodes resident
+ * workgroups do (a cooperative launch, outside stream capture), above that each day is a
+ * launch.  If the resident workgroups cannot all run for 10 s the rows they did not reach
+ * hold NaN.
+ *
  * Arrays are device pointers (float32, node-major rows of n).  All work is
  * queued on `hip_stream` (NULL = default stream).  Returns 0 or a negative
  * LP_ERR_* code of lp_step.h.

@@ -10,9 +10,9 @@ per-node r0_scalars, the gravity network parameters k, a, b, c
 Node compartments are aggregated from an ABM population at day 0 and rolled
 forward deterministically (expected exposures, daily E -> I and I -> R exits at
 the mean durations).  ``MeanFieldRollout`` is a torch.autograd.Function whose
-forward and hand-written adjoint run in liblpstep.so (lp_meanfield.h); it keeps
-the state only every ``checkpoint`` days and recomputes each segment forward
-before its adjoint.  ``rollout_reference`` is the same rollout in plain PyTorch
+forward and hand-written adjoint run in liblpstep.so (lp_meanfield.h); a rollout
+too large to keep whole (KEEP_BYTES) keeps the state only every ``checkpoint``
+days and recomputes each segment forward before its adjoint.  ``rollout_reference`` is the same rollout in plain PyTorch
 ops, for autograd and finite-difference checks.
 """
 
@@ -41,6 +41,10 @@ class LPMFModel(ctypes.Structure):
         ("pad", ctypes.c_float),
     ]
 
+
+# a rollout whose S, I, m and g trajectories (16 bytes a node and day) take no more than
+# this keeps them for its adjoint; a larger one is checkpointed and recomputed
+KEEP_BYTES = 256 << 20
 
 _mf = None
 
@@ -86,17 +90,24 @@ class MeanFieldRollout(torch.autograd.Function):
                           inv_tau_i=float(inv_tau_i))
         stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
         inc = torch.empty((T, n), **f32)
-        state = [x.detach().to(**f32).reshape(1, n).contiguous() for x in (S0, E0, I0)]
+        # a rollout whose trajectories are small is kept whole for the adjoint: one call over
+        # all its days, nothing recomputed
+        grad = any(ctx.needs_input_grad)
+        keep_all = checkpoint > 0 and 0 < 16 * T * n <= KEEP_BYTES
+        state = [x.detach().to(**f32).reshape(1, n) for x in (S0, E0, I0)]
         checkpoints = []
-        for t0 in range(0, T, checkpoint):
-            t1 = min(T, t0 + checkpoint)
-            checkpoints.append((t0, t1, [x.clone() for x in state]))
+        for t0 in range(0, T, T if keep_all else checkpoint):
+            t1 = T if keep_all else min(T, t0 + checkpoint)
             traj = [torch.empty((t1 - t0 + 1, n), **f32) for _ in range(3)]
             for tr, x in zip(traj, state):
                 tr[0].copy_(x[0])
+            saves = [torch.empty((T, n), **f32) for _ in range(2)] if keep_all and grad else [None, None]
             _check(_lib().lp_mf_days(ctypes.byref(model), t0, t1, _p(traj[0]), _p(traj[1]), _p(traj[2]),
-                                     _p(inc[t0:t1]), None, None, stream), "lp_mf_days")
-            state = [tr[-1:].clone() for tr in traj]
+                                     _p(inc[t0:t1]), _p(saves[0]), _p(saves[1]), stream), "lp_mf_days")
+            if grad:
+                kept = (traj[0], traj[2], *saves) if keep_all else None
+                checkpoints.append((t0, t1, [tr[:1].clone() for tr in traj] if kept is None else None, kept))
+            state = [tr[-1:] for tr in traj]
         ctx.model = model
         ctx.keepalive = (net, net_t, keep, r0s, rho, inv_pop, season)
         ctx.checkpoints = checkpoints
@@ -113,20 +124,22 @@ class MeanFieldRollout(torch.autograd.Function):
         g_inc = g_inc.to(**f32).contiguous()
         r0_bar = torch.zeros(n, **f32)
         net_bar = torch.zeros((n, n), **f32)
-        season_part = torch.zeros((T, n), **f32)
+        season_part = torch.empty((T, n), **f32)     # every row is written
         aS, aE, aI = (torch.zeros(n, **f32) for _ in range(3))
-        work = torch.zeros(2 * n, **f32)
-        for t0, t1, state in reversed(ctx.checkpoints):
-            L = t1 - t0
-            traj = [torch.empty((L + 1, n), **f32) for _ in range(3)]
-            for tr, x in zip(traj, state):
-                tr[0].copy_(x[0])
-            inc = torch.empty((L, n), **f32)
-            msave, gsave = torch.empty((L, n), **f32), torch.empty((L, n), **f32)
-            _check(_lib().lp_mf_days(ctypes.byref(model), t0, t1, _p(traj[0]), _p(traj[1]), _p(traj[2]), _p(inc),
-                                     _p(msave), _p(gsave), stream), "lp_mf_days")
-            _check(_lib().lp_mf_adjoint_days(ctypes.byref(model), t0, t1, _p(traj[0]), _p(traj[2]), _p(msave),
-                                             _p(gsave), _p(g_inc[t0:t1]), _p(aS), _p(aE), _p(aI), _p(r0_bar),
+        work = torch.empty(2 * n, **f32)
+        for t0, t1, state, kept in reversed(ctx.checkpoints):
+            if kept is None:
+                L = t1 - t0
+                traj = [torch.empty((L + 1, n), **f32) for _ in range(3)]
+                for tr, x in zip(traj, state):
+                    tr[0].copy_(x[0])
+                inc = torch.empty((L, n), **f32)
+                msave, gsave = torch.empty((L, n), **f32), torch.empty((L, n), **f32)
+                _check(_lib().lp_mf_days(ctypes.byref(model), t0, t1, _p(traj[0]), _p(traj[1]), _p(traj[2]), _p(inc),
+                                         _p(msave), _p(gsave), stream), "lp_mf_days")
+                kept = (traj[0], traj[2], msave, gsave)
+            _check(_lib().lp_mf_adjoint_days(ctypes.byref(model), t0, t1, *(_p(x) for x in kept),
+                                             _p(g_inc[t0:t1]), _p(aS), _p(aE), _p(aI), _p(r0_bar),
                                              _p(net_bar), _p(season_part[t0:t1]), _p(work), stream),
                    "lp_mf_adjoint_days")
         season_bar = season_part.sum(dim=1)
