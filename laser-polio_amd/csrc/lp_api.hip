@@ -693,7 +693,7 @@ int lp_init_population(lp_ctx* c, const lp_init_sim* sims, int32_t n_sims, const
   if (n_inf > 0) HIPCHK(c, hipMalloc(&inf_d, sizeof(int64_t) * n_inf));
   HIPCHK(c, hipMemcpyAsync(specs_d, sims, sizeof(lp_init_sim) * n_sims, hipMemcpyHostToDevice, c->stream));
   if (n_inf > 0) HIPCHK(c, hipMemcpyAsync(inf_d, infected, sizeof(int64_t) * n_inf, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(lp::k_init, dim3(c->n_spans), dim3(lp::WG), 0, c->stream, c->d, specs_d);
+  hipLaunchKernelGGL(lp::k_init, dim3(tile_grid(c)), dim3(lp::WG), 0, c->stream, c->d, specs_d);
   if (n_inf > 0)
     hipLaunchKernelGGL(lp::k_init_infected, dim3(grid_of(n_inf, 256) < 4096 ? grid_of(n_inf, 256) : 4096), dim3(256), 0,
                        c->stream, c->d, inf_d, n_inf);
