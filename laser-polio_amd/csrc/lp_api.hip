@@ -125,7 +125,11 @@ struct lp_ctx {
   int64_t time_launches = 0;
   double time_ms = 0.0;
   lp_gravity_spec* net_specs = nullptr;            // lp_build_network inputs (n_sims), allocated on first use
-  double* net_scratch = nullptr;                   // row scales and 1 / S^c per node
+  lp_gravity_spec* net_specs_h = nullptr;          // their pinned staging copy
+  double* net_scratch = nullptr;                   // NetScratch's per-node and per-simulation values
+  double* net_w = nullptr;                         // every entry in float64 (null: no room)
+  int64_t net_len = 0;                             // entries of network_t
+  int32_t max_sim_nodes = 0;                       // nodes of the largest simulation
 };
 
 namespace {
@@ -463,8 +467,10 @@ int lp_prepare(lp_ctx* c) {
       return fail(c, LP_ERR_ARG, "bad node segment " + std::to_string(n));
     if (nsim[n] < 0 || nsim[n] >= S) return fail(c, LP_ERR_ARG, "bad node_sim " + std::to_string(n));
   }
+  c->net_len = net_len;
   for (int s = 0; s < S; ++s) {
     const lp_sim_params& p = sims[s];
+    c->max_sim_nodes = std::max(c->max_sim_nodes, (int32_t)p.n_nodes);
     if (p.n_nodes <= 0 || p.node_begin < 0 || p.node_begin + p.n_nodes > N)
       return fail(c, LP_ERR_ARG, "bad sim node range " + std::to_string(s));
     for (int n = p.node_begin; n < p.node_begin + p.n_nodes; ++n)
@@ -555,9 +561,7 @@ int lp_prepare(lp_ctx* c) {
   d.mix_buf = nullptr;
   if (g.mix_mode == 1) {
     if ((rc = alloc(c, &d.mix_buf, (size_t)N * LP_MAX_STRAINS))) return rc;
-    int max_n = 0;
-    for (const auto& p : sims) max_n = std::max(max_n, (int)p.n_nodes);
-    c->mix_tiles = (max_n + 15) / 16;
+    c->mix_tiles = (c->max_sim_nodes + 15) / 16;
   }
   if ((rc = alloc(c, &d.sim_cases, (size_t)S))) return rc;
   if ((rc = alloc(c, &d.ninfo, (size_t)N))) return rc;
@@ -714,28 +718,33 @@ int lp_build_network(lp_ctx* c, const lp_gravity_spec* specs, int32_t n_sims, co
   if (!c || !specs || !pop || !dist) return LP_ERR_ARG;
   if (!c->prepared) return fail(c, LP_ERR_STATE, "lp_build_network before lp_prepare");
   if (n_sims != c->cfg.n_sims) return fail(c, LP_ERR_ARG, "lp_build_network: one lp_gravity_spec per simulation");
-  int max_n = 0;
   for (int s = 0; s < n_sims; ++s) {
     const lp_gravity_spec& g = specs[s];
     if (!(g.max_rowsum >= 0.0) || !(g.k >= 0.0)) return fail(c, LP_ERR_ARG, "lp_build_network: bad spec for sim " + std::to_string(s));
   }
-  std::vector<lp_sim_params> sp((size_t)n_sims);
-  HIPCHK(c, hipMemcpyAsync(sp.data(), c->d.sims, sizeof(lp_sim_params) * n_sims, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  for (const auto& p : sp) max_n = std::max(max_n, (int)p.n_nodes);
+  const size_t N = (size_t)c->cfg.n_nodes;
   int rc;
-  if (!c->net_specs && (rc = alloc(c, &c->net_specs, (size_t)n_sims))) return rc;
-  if (!c->net_scratch && (rc = alloc(c, &c->net_scratch, 2 * (size_t)c->cfg.n_nodes))) return rc;
-  HIPCHK(c, hipMemcpyAsync(c->net_specs, specs, sizeof(lp_gravity_spec) * n_sims, hipMemcpyHostToDevice, c->stream));
-  double* scale = c->net_scratch;
-  double* inv_sc = c->net_scratch + c->cfg.n_nodes;
-  hipLaunchKernelGGL(lp::k_net_rows, dim3(c->cfg.n_nodes), dim3(lp::WG), 0, c->stream, c->d, c->net_specs, pop, dist, scale,
-                     inv_sc);
+  if (!c->net_specs) {
+    // kept for the context's later builds; without room for every entry in float64 the
+    // last pass takes the powers again
+    if ((rc = alloc(c, &c->net_scratch, 3 * N + (size_t)n_sims))) return rc;
+    void* w = nullptr;
+    if (hipMalloc(&w, (size_t)c->net_len * sizeof(double)) == hipSuccess) c->allocs.push_back(w);
+    else (void)hipGetLastError();
+    c->net_w = static_cast<double*>(w);
+    HIPCHK(c, hipHostMalloc(reinterpret_cast<void**>(&c->net_specs_h), sizeof(lp_gravity_spec) * n_sims, hipHostMallocDefault));
+    if ((rc = alloc(c, &c->net_specs, (size_t)n_sims))) return rc;
+  }
+  std::memcpy(c->net_specs_h, specs, sizeof(lp_gravity_spec) * n_sims);
+  HIPCHK(c, hipMemcpyAsync(c->net_specs, c->net_specs_h, sizeof(lp_gravity_spec) * n_sims, hipMemcpyHostToDevice, c->stream));
+  double* x = c->net_scratch;
+  const lp::NetScratch ns{x, x + N, x + 2 * N, x + 3 * N, c->net_w};
+  const int max_n = c->max_sim_nodes;
+  hipLaunchKernelGGL(lp::k_net_pow, dim3(n_sims, grid_of(max_n, lp::WG)), dim3(lp::WG), 0, c->stream, c->d, c->net_specs, pop, ns);
+  hipLaunchKernelGGL(lp::k_net_rows, dim3(c->cfg.n_nodes), dim3(lp::WG), 0, c->stream, c->d, c->net_specs, dist, ns);
   const int tiles = (max_n + lp::NET_TILE - 1) / lp::NET_TILE;
-  hipLaunchKernelGGL(lp::k_net_tiles, dim3(tiles * tiles, n_sims), dim3(lp::WG), 0, c->stream, c->d, c->net_specs, pop,
-                     dist, scale, inv_sc);
+  hipLaunchKernelGGL(lp::k_net_tiles, dim3(tiles * tiles, n_sims), dim3(lp::WG), 0, c->stream, c->d, c->net_specs, dist, ns);
   HIPCHK(c, hipGetLastError());
-  // the specs are copied before the call returns (pageable host memory)
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return LP_OK;
 }
@@ -838,6 +847,7 @@ void lp_destroy(lp_ctx* c) {
       if (c->graph[k][j]) (void)hipGraphExecDestroy(c->graph[k][j]);
   for (hipEvent_t e : c->ev) (void)hipEventDestroy(e);
   for (void* p : c->allocs) (void)hipFree(p);
+  if (c->net_specs_h) (void)hipHostFree(c->net_specs_h);
   if (c->own_stream && c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
 }
