@@ -101,6 +101,7 @@ struct lp_ctx {
   bool own_stream = false;
   bool prepared = false;
   int32_t n_spans = 0;
+  int32_t n_tiles = 0;
   int32_t tpw = 4;
   int32_t agent_grid = 1;
   int32_t ei_grid = 2048, sample_grid = 2048;     // launch shapes of the list pass and the sampler
@@ -242,9 +243,6 @@ void launch_agents_u(lp_ctx* c, hipStream_t s, int kind, int mask) {
   }
 }
 
-// Grid of the passes with one workgroup per tile: span << tpw_sh | tile of the span.
-int tile_grid(const lp_ctx* c) { return c->n_spans << c->d.tpw_sh; }
-
 // Day kinds that process the E / I list; afterwards the records of listed agents
 // keep the timers of when they entered the list until enqueue_actualize.
 bool list_kind(int kind) { return kind == lp::KIND_PLAIN_LIST || kind >= lp::KIND_FULL_LIST; }
@@ -262,7 +260,7 @@ void enqueue_actualize(lp_ctx* c) {
 // Bound columns <- device-held state: agent records and actual ri_timer values.
 void enqueue_sync_columns(lp_ctx* c) {
   enqueue_actualize(c);
-  hipLaunchKernelGGL(lp::k_unpack, dim3(tile_grid(c)), dim3(lp::WG), 0, c->stream, c->d);
+  hipLaunchKernelGGL(lp::k_unpack, dim3(c->n_tiles), dim3(lp::WG), 0, c->stream, c->d);
   hipLaunchKernelGGL(lp::k_ri_sync, dim3(c->n_spans), dim3(lp::WG), 0, c->stream, c->d);
   hipLaunchKernelGGL(lp::k_set_ri_ref, dim3(1), dim3(64), 0, c->stream, c->d, -2);
 }
@@ -297,7 +295,7 @@ void enqueue_recount(lp_ctx* c, int32_t t, int32_t until, bool lists, bool ri) {
   if (c->rec_dirty) enqueue_sync_columns(c);   // the pass reads the columns
   hipLaunchKernelGGL(lp::k_recount_begin, dim3(grid_of(n, lp::WG)), dim3(lp::WG), 0, c->stream, c->d, ri ? 1 : 0,
                      t, until);
-  hipLaunchKernelGGL(lp::k_recount, dim3(tile_grid(c)), dim3(lp::WG), 0, c->stream, c->d, lists ? 1 : 0);
+  hipLaunchKernelGGL(lp::k_recount, dim3(c->n_tiles), dim3(lp::WG), 0, c->stream, c->d, lists ? 1 : 0);
   c->recount_pending = false;
   c->rec_dirty = true;
   c->rec_actual = true;
@@ -528,10 +526,17 @@ int lp_prepare(lp_ctx* c) {
     // CU); above that 512 threads held to 6 waves per SIMD (three a CU)
     c->finish_wide = N <= cus;
   }
-  int4* spans_d; int32_t* nspan_d;
+  std::vector<int32_t> tiles;
+  for (size_t i = 0; i < spans.size(); ++i)
+    for (int u = 0; u < spans[i].z; ++u) tiles.push_back((int32_t)i << d.tpw_sh | u);   // below 2^26: 2^22 tiles, 16 a span
+  c->n_tiles = (int32_t)tiles.size();
+  int4* spans_d; int32_t *nspan_d, *tiles_d;
   int rc;
   if ((rc = alloc(c, &spans_d, spans.size()))) return rc;
   if ((rc = alloc(c, &nspan_d, N + 1))) return rc;
+  if ((rc = alloc(c, &tiles_d, tiles.size()))) return rc;
+  HIPCHK(c, hipMemcpyAsync(tiles_d, tiles.data(), tiles.size() * 4, hipMemcpyHostToDevice, c->stream));
+  d.tiles = tiles_d;
   HIPCHK(c, hipMemcpyAsync(spans_d, spans.data(), spans.size() * sizeof(int4), hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipMemcpyAsync(nspan_d, nspan.data(), (N + 1) * 4, hipMemcpyHostToDevice, c->stream));
   d.spans = spans_d; d.node_span_begin = nspan_d;
@@ -697,7 +702,7 @@ int lp_init_population(lp_ctx* c, const lp_init_sim* sims, int32_t n_sims, const
   if (n_inf > 0) HIPCHK(c, hipMalloc(&inf_d, sizeof(int64_t) * n_inf));
   HIPCHK(c, hipMemcpyAsync(specs_d, sims, sizeof(lp_init_sim) * n_sims, hipMemcpyHostToDevice, c->stream));
   if (n_inf > 0) HIPCHK(c, hipMemcpyAsync(inf_d, infected, sizeof(int64_t) * n_inf, hipMemcpyHostToDevice, c->stream));
-  hipLaunchKernelGGL(lp::k_init, dim3(tile_grid(c)), dim3(lp::WG), 0, c->stream, c->d, specs_d);
+  hipLaunchKernelGGL(lp::k_init, dim3(c->n_tiles), dim3(lp::WG), 0, c->stream, c->d, specs_d);
   if (n_inf > 0)
     hipLaunchKernelGGL(lp::k_init_infected, dim3(grid_of(n_inf, 256) < 4096 ? grid_of(n_inf, 256) : 4096), dim3(256), 0,
                        c->stream, c->d, inf_d, n_inf);

@@ -173,9 +173,8 @@ __device__ int32_t init_age(const lp_init_sim& sp, uint64_t seed, uint64_t slot)
 // logarithms, roots and cosines per agent): 4.9 ms for 269 M slots, of which 2.0 ms are
 // the 32 bytes a slot; 7.5 ms before, 5.4 with the shorter Philox rounds alone.
 __global__ void __launch_bounds__(WG) k_init(Dev d, const lp_init_sim* specs) {
-  const int4 span = d.spans[blockIdx.x >> d.tpw_sh];
-  const int u = blockIdx.x & ((1 << d.tpw_sh) - 1);
-  if (u >= span.z) return;
+  const int tile = d.tiles[blockIdx.x], u = tile & ((1 << d.tpw_sh) - 1);
+  const int4 span = d.spans[tile >> d.tpw_sh];
   const int node = span.x, sim = span.w;
   const lp_sim_params& simp = d.sims[sim];
   const lp_init_sim& sp = specs[sim];

@@ -109,6 +109,7 @@ struct Dev {
   int32_t* day;   // [8] tick, end of the lp_run_days call, unused x2, the day record (today())
   int32_t* stop_day; int32_t* err;
   const int4* spans; const int32_t* node_span_begin;
+  const int32_t* tiles;    // every tile of every span: span << tpw_sh | tile of the span
   int64_t* partials; int64_t* chunk_sum;
   int64_t* nb_begin; int32_t* births;
   int64_t* node_tally; int32_t* potp_run; int32_t* p_run;
@@ -734,8 +735,7 @@ __global__ void __launch_bounds__(WG) k_recount_begin(Dev d, int ri, int32_t t, 
   node_info(d, i);
 }
 
-// One workgroup per tile (blockIdx.x = span << tpw_sh | tile of the span), one quad of slots per
-// thread: the agent records from the columns; per chunk the weight of its S agents and
+// One workgroup per tile, one quad of slots per thread: the agent records from the columns; per chunk the weight of its S agents and
 // the earliest death date of its live ones; per span its weight; per node #S, #S with
 // positive weight, #R, the potentially paralysed and the paralysed; with `lists` the node's
 // E / I list of today (timers as of the start of today); the RI candidates of the next RI
@@ -745,9 +745,8 @@ __global__ void __launch_bounds__(WG) k_recount_begin(Dev d, int ri, int32_t t, 
 // (A pass per span that also ran the day took 2.7 ms there and a separate record pass
 // 3.2 ms; at 5.4 M slots, 330 workgroups of 16 tiles each, 280 and 50 us against 61 us.)
 __global__ void __launch_bounds__(WG) k_recount(Dev d, int lists) {
-  const int4 span = d.spans[blockIdx.x >> d.tpw_sh];
-  const int u = blockIdx.x & ((1 << d.tpw_sh) - 1);
-  if (u >= span.z) return;
+  const int tile = d.tiles[blockIdx.x], u = tile & ((1 << d.tpw_sh) - 1);
+  const int4 span = d.spans[tile >> d.tpw_sh];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int node = span.x, sim = span.w;
   const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)tid * 4;
@@ -828,7 +827,7 @@ __global__ void __launch_bounds__(WG) k_recount(Dev d, int lists) {
          : tid < 6 ? (int64_t)((s_p[w] >> (16 * (tid - 4))) & 0xffffu) : (int64_t)((s_l[w] >> (16 * (tid - 6))) & 0xffff);
     if (v != 0) {
       if (tid == 0)
-        atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(blockIdx.x >> d.tpw_sh) * NPART + P_SW),
+        atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(tile >> d.tpw_sh) * NPART + P_SW),
                   (unsigned long long)v);
       else if (tid < 4)
         atomicAdd(reinterpret_cast<unsigned long long*>(d.node_carry + (size_t)node * 3 + tid - 1), (unsigned long long)v);
@@ -862,10 +861,10 @@ __global__ void __launch_bounds__(WG) k_recount(Dev d, int lists) {
 // held yet).  Bound by HBM: 27 bytes a live slot in 16-, 8- and 4-byte accesses, 1.25 ms
 // for 227 M agents in 269 M slots (4.9 TB/s; byte stores over every slot took 2.6 ms).
 __global__ void __launch_bounds__(WG) k_unpack(Dev d) {
-  const int4 span = d.spans[blockIdx.x >> d.tpw_sh];
-  const int u = blockIdx.x & ((1 << d.tpw_sh) - 1);
+  const int tile = d.tiles[blockIdx.x], u = tile & ((1 << d.tpw_sh) - 1);
+  const int4 span = d.spans[tile >> d.tpw_sh];
   const int64_t i0 = ((int64_t)span.y + u) * LP_TILE + (int64_t)threadIdx.x * 4;
-  if (u >= span.z || i0 >= d.live_end[span.x]) return;
+  if (i0 >= d.live_end[span.x]) return;
   const int64_t q0 = i0 >> 2;
   uint4 r[4];
 #pragma unroll
