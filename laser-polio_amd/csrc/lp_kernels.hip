@@ -1011,7 +1011,13 @@ __global__ void __launch_bounds__(WG) k_plain(Dev d, int mask) {
 // pieces of EI_PIECE entries of one node (ei_piece_off) in turn and adds the
 // piece's tallies to node_acc with one atomic per field; k_node_reduce reads
 // them in place of the span partials.  Cost: proportional to the E and I
-// agents, not to the population.
+// agents, not to the population.  With many of them the traffic bounds it (5.8 M
+// agents 70 us, 145 on VD days, which read each one's date of death), with few the chain
+// from the day record over the piece scan, the node, the entries and their records to
+// the place in tomorrow's list (8 us).  So a piece's reads of one kind go out together:
+// the transitions of its four entries per lane first (entries alone), then the records of
+// its paralysis rolls beside the atomic for its survivors' places (one entry after the
+// other: 64 replicates at their peak 91 -> 83 us, the year 70.8 -> 69.9 ms).
 
 // Exclusive prefix over n in [0, N) of cnt(n), by every thread of one workgroup:
 // emit(n, prefix) for each n; returns the total.  Each pass takes 4 * WG nodes, 4
@@ -1091,14 +1097,7 @@ __global__ void __launch_bounds__(WG) k_ei(Dev d, int mask) {
     total = d.ei_piece_off[N];   // planned by k_ei_plan
   }
   for (int32_t p = gw; p < total; p += nw) {
-    int n;
-    if (lds) {
-      int a = 0, b = N;   // largest n with s_off[n] <= p
-      while (b - a > 1) { const int m = (a + b) >> 1; if (s_off[m] <= p) a = m; else b = m; }
-      n = a;
-    } else {
-      n = find_piece_node(d.ei_piece_off, N, p, lane);
-    }
+    int n = lds ? find_piece_node(s_off, N, p, lane) : find_piece_node(d.ei_piece_off, N, p, lane);
     n = __builtin_amdgcn_readfirstlane(n);   // the same in every lane: scalar loads of the node's data
     const NodeInfo ni = d.ninfo[n];
     const int32_t cnt = d.ei_cnt[(size_t)cur * N + n];
@@ -1129,7 +1128,9 @@ __global__ void __launch_bounds__(WG) k_ei(Dev d, int mask) {
     // tallies: E and I counts per strain in 16-bit fields, I->R / new potentially
     // paralysed / new paralysed in 16-bit fields, infectious weight per strain
     int64_t e_pk = 0, i_pk = 0, misc = 0, ib0 = 0, ib1 = 0, ib2 = 0, ib3 = 0;
-    uint32_t surv = 0;
+    uint32_t surv = 0, par = 0;
+    // today's transitions (model.py:419-452).  Who stays in E or I follows from the
+    // entries alone; only the paralysis roll reads its agent's record.
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       uint4 e = ent[q];
@@ -1141,10 +1142,9 @@ __global__ void __launch_bounds__(WG) k_ei(Dev d, int mask) {
       if (dd[q] <= t) { ei_actual_timers(d, e, t); continue; }   // dies today: the VD pass takes it
       const int k = ent_strain(e);
       if (do_ds && ent_event(e) <= t) {
-        // today's transitions (model.py:419-452)
         uint16_t* hw = reinterpret_cast<uint16_t*>(d.rec + slot);
         int32_t i_end = (int32_t)e.z, p_day = ent_day(e);
-        bool pend = ent_pend(e), to_par = false;
+        bool pend = ent_pend(e);
         const bool s0 = k == 0;
         const int s_in = sa;
         if (sa == 1) {                                    // E -> I: the exposure timer reads 0
@@ -1153,63 +1153,70 @@ __global__ void __launch_bounds__(WG) k_ei(Dev d, int mask) {
           p_day = s0 ? t + (int32_t)(e.z >> 16) : (int32_t)DAY_NONE;
           hw[0] = 0;
         }
-        if (pend && p_day <= t) {                         // the paralysis timer reads 0 with pp -1
-          pend = false;
-          int8_t pp = 0;
-          if (*rec_byte(d, slot, RB_IPV) == 0) {          // not ipv_protected
-            pp = 1;
-            misc += 1ll << 16;
-            const uint4 o = draw(ec.seed, (uint64_t)((int64_t)slot - ec.slot_base), t, ST_PARALYSIS);
-            if ((uint64_t)o.x < ec.thr_paralysis) { to_par = true; misc += 1ll << 32; }
-          }
-          *rec_byte(d, slot, RB_PP) = pp;
-        }
+        if (pend && p_day <= t) { pend = false; par |= 1u << q; }   // the paralysis timer reads 0 with pp -1
         if (i_end <= t) {                                 // I -> R: the infection timer reads 0
           sa = 3;
           misc += 1;
           hw[1] = 0;
           if (s0) hw[2] = (uint16_t)timer_left(p_day, t + 1);   // stops after today's count-down
         }
-        if (to_par) *rec_byte(d, slot, RB_PARALYZED) = 1;
         if (sa != s_in) d.state[slot] = (int8_t)sa;
         if (sa == 2) e = make_uint4(slot, ent_flags(2, k, pend, p_day), (uint32_t)i_end, e.w);
       }
       if (sa != 1 && sa != 2) continue;
       surv |= 1u << q;
       ent[q] = e;
-      if (do_tally) {                                     // tx_step_prep / count_SEIRP tally of E and I
-        if (sa == 1) {
+    }
+    // the records of the paralysis rolls and the place in the next day's list (one atomic
+    // per piece), on their way together
+    int8_t ipv[4] = {1, 1, 1, 1};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) if ((par >> q) & 1u) ipv[q] = *rec_byte(d, ent[q].x, RB_IPV);
+    int rank[4], tot = 0, base = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint64_t mk = __ballot((surv >> q) & 1u);
+      rank[q] = tot + __popcll(mk & ((1ull << lane) - 1ull));
+      tot += __popcll(mk);
+    }
+    if (tot && lane == 0) base = atomicAdd(d.ei_cnt + (size_t)nxt * N + n, tot);
+    if (do_tally) {                                       // tx_step_prep / count_SEIRP tally of E and I
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (!((surv >> q) & 1u)) continue;
+        const uint4 e = ent[q];
+        const int k = ent_strain(e);
+        if (ent_state(e) == 1) {
           e_pk += 1ll << (16 * k);
         } else {
           i_pk += 1ll << (16 * k);
           int64_t wv = (int64_t)e.w;
           if (e.w == W_REC) {
             const float rk = k == 0 ? ec.r0k[0] : k == 1 ? ec.r0k[1] : k == 2 ? ec.r0k[2] : ec.r0k[3];
-            wv = weight_q24(__uint_as_float(d.rec[slot].z) * rk);
+            wv = weight_q24(__uint_as_float(d.rec[e.x].z) * rk);
           }
           ib0 += k == 0 ? wv : 0; ib1 += k == 1 ? wv : 0; ib2 += k == 2 ? wv : 0; ib3 += k == 3 ? wv : 0;
         }
       }
     }
-    // survivors -> next day's list: one atomic per piece
-    {
-      uint64_t mk[4];
-      int rank[4], tot = 0;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        mk[q] = __ballot((surv >> q) & 1u);
-        rank[q] = tot + __popcll(mk[q] & ((1ull << lane) - 1ull));
-        tot += __popcll(mk[q]);
+    for (int q = 0; q < 4; ++q) {
+      if (!((par >> q) & 1u)) continue;
+      const uint32_t slot = ent[q].x;
+      if (ipv[q] == 0) {                                  // not ipv_protected
+        misc += 1ll << 16;
+        const uint4 o = draw(ec.seed, (uint64_t)((int64_t)slot - ec.slot_base), t, ST_PARALYSIS);
+        if ((uint64_t)o.x < ec.thr_paralysis) { *rec_byte(d, slot, RB_PARALYZED) = 1; misc += 1ll << 32; }
       }
-      if (tot) {
-        int base = 0;
-        if (lane == 0) base = atomicAdd(d.ei_cnt + (size_t)nxt * N + n, tot);
-        base = __shfl(base, 0, 64);
-        uint4* Ln = d.ei_list + (size_t)nxt * (size_t)d.capacity + ni.seg_begin;
+      *rec_byte(d, slot, RB_PP) = ipv[q] == 0 ? 1 : 0;
+    }
+    // survivors -> next day's list
+    if (tot) {
+      base = __builtin_amdgcn_readfirstlane(base);
+      uint4* Ln = d.ei_list + (size_t)nxt * (size_t)d.capacity + ni.seg_begin;
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
-          if ((surv >> q) & 1u) Ln[base + rank[q]] = ent[q];
-      }
+      for (int q = 0; q < 4; ++q)
+        if ((surv >> q) & 1u) Ln[base + rank[q]] = ent[q];
     }
     if (stopped) continue;
     // the piece's tallies -> node_acc (lanes 0..14 one field each)
