@@ -647,7 +647,8 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
     }
     if (list_kind(kind)) c->rec_actual = false;
     else enqueue_actualize(c);
-    c->list_tick = t + 1;   // every day kind run here completes the next tick's list
+    // the day completes the next tick's list, unless its dense pass reads no E or I agent
+    c->list_tick = host_stage_flags(c->day_flags_h[t], LP_STAGE_ALL) & (LP_DAY_DS | LP_DAY_TX) ? t + 1 : -1;
     if (use_graph && !c->timing && !first && c->stream != nullptr) {
       // the following days of the same list kind (each completes the next one's list,
       // so they need nothing from the host in between) join this day's graph: 2^j days
@@ -662,7 +663,7 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
       HIPCHK(c, hipGraphLaunch(c->graph[kind][j], c->stream));
       c->rec_dirty = true;   // as enqueue_day marks it: the columns are behind the records
       t += run - 1;
-      c->list_tick = t + 1;
+      if (run > 1) c->list_tick = t + 1;   // (of the list kinds)
     } else {
       if ((rc = enqueue_day(c, t, kind, LP_STAGE_ALL, 1, true, first, t_end))) return rc;
     }
