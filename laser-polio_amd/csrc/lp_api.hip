@@ -304,7 +304,8 @@ void enqueue_recount(lp_ctx* c, int32_t t, int32_t until, bool lists, bool ri) {
 // The kernel sequence of one tick.  kind: agent-pass variant; mask: stages;
 // tx_adjust: apply today's transmission exposures to the log; advance: move
 // the day counter at the end; begin: the day begins here, in a call that runs to tick
-// `until` (0: stage calls), not at the end of the day before.
+// `until` (0: stage calls), not at the end of the day before.  Days of the list kinds (the
+// whole day, advanced) end in k_finish, the others in k_day_end.
 int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool advance, bool begin, int32_t until = 0) {
   const Dev& d = c->d;
   const int N = c->cfg.n_nodes;
@@ -342,13 +343,15 @@ int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool ad
     const size_t off_lds = (N + 1 <= lp::LDS_OFF_MAX) ? (size_t)(N + 1) * sizeof(int64_t) : 0;
     if (!off_lds) hipLaunchKernelGGL(lp::k_plan, dim3(1), dim3(lp::WG), 0, s, d, 1);
     hipLaunchKernelGGL(lp::k_sample, dim3(c->sample_grid), dim3(lp::WG), off_lds, s, d);
+    // the days of the list kinds, which only lp_run_days runs, end in k_finish itself
+    const int end = list_kind(kind) ? 1 : 0;
     if (c->finish_wide)
-      hipLaunchKernelGGL((lp::k_finish<1024, 4>), dim3(N), dim3(1024), 0, s, d);
+      hipLaunchKernelGGL((lp::k_finish<1024, 4>), dim3(N), dim3(1024), 0, s, d, end);
     else
-      hipLaunchKernelGGL((lp::k_finish<512, 6>), dim3(N), dim3(512), 0, s, d);
+      hipLaunchKernelGGL((lp::k_finish<512, 6>), dim3(N), dim3(512), 0, s, d, end);
   }
   // (stages before transmission leave it nothing to do)
-  if (advance || (mask & (LP_STAGE_TRANSMISSION | LP_STAGE_LOG)))
+  if (!list_kind(kind) && (advance || (mask & (LP_STAGE_TRANSMISSION | LP_STAGE_LOG))))
     hipLaunchKernelGGL(lp::k_day_end, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask, tx_adjust, advance ? 1 : 0);
   HIPCHK(c, hipGetLastError());
   c->rec_dirty = true;
@@ -541,7 +544,7 @@ int lp_prepare(lp_ctx* c) {
   HIPCHK(c, hipMemcpyAsync(nspan_d, nspan.data(), (N + 1) * 4, hipMemcpyHostToDevice, c->stream));
   d.spans = spans_d; d.node_span_begin = nspan_d;
   const int64_t nch = g.capacity / LP_CHUNK + 1;
-  if ((rc = alloc(c, &d.day, 8))) return rc;   // t, until, -, -, then the day record (16-byte aligned)
+  if ((rc = alloc(c, &d.day, 12))) return rc;   // t, until, -, -, then the two day records (16-byte aligned)
   if ((rc = alloc(c, &d.stop_day, S))) return rc;
   if ((rc = alloc(c, &d.err, 4))) return rc;
   if ((rc = alloc(c, &d.partials, (size_t)c->n_spans * lp::NPART))) return rc;
@@ -607,6 +610,12 @@ int lp_prepare(lp_ctx* c) {
     d.ri_cnt = rc_d;
     if ((rc = alloc(c, &d.ri_ref, 2))) return rc;
   }
+  lp::CloseField close_tab[128];
+  lp::close_fields(d, close_tab);
+  lp::CloseField* close_d = nullptr;
+  if ((rc = alloc(c, &close_d, 128))) return rc;
+  HIPCHK(c, hipMemcpyAsync(close_d, close_tab, sizeof close_tab, hipMemcpyHostToDevice, c->stream));
+  d.close_tab = close_d;
   std::vector<int32_t> stop(S, INT_MAX);
   HIPCHK(c, hipMemcpyAsync(d.stop_day, stop.data(), S * 4, hipMemcpyHostToDevice, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -620,8 +629,9 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
   if (t_begin < 0 || t_end > c->cfg.nt || t_begin > t_end) return fail(c, LP_ERR_ARG, "bad tick range");
   if (t_begin == t_end) return LP_OK;
   first_run(c, t_begin);
-  // inside the call each day's k_day_end begins the next day; only the first is begun here
+  // inside the call each day's end begins the next day; only the first is begun here
   bool first = true;
+  bool ahead = false;   // the day before ended in k_finish: k_ei's record is a day ahead of the others
   int rc;
   int32_t t = t_begin;
   if (t == 0) {
@@ -645,8 +655,13 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
       if (kind == lp::KIND_PLAIN) kind = lp::KIND_PLAIN_LIST;
       else if (kind >= lp::KIND_FULL && kind < lp::KIND_PLAIN_LIST) kind = lp::KIND_FULL_LIST + kind - lp::KIND_FULL;
     }
-    if (list_kind(kind)) c->rec_actual = false;
-    else enqueue_actualize(c);
+    if (list_kind(kind)) {
+      c->rec_actual = false;
+    } else {
+      enqueue_actualize(c);
+      if (ahead) hipLaunchKernelGGL(lp::k_advance, dim3(1), dim3(1), 0, c->stream, c->d);
+    }
+    ahead = list_kind(kind);
     // the day completes the next tick's list, unless its dense pass reads no E or I agent
     c->list_tick = host_stage_flags(c->day_flags_h[t], LP_STAGE_ALL) & (LP_DAY_DS | LP_DAY_TX) ? t + 1 : -1;
     if (use_graph && !c->timing && !first && c->stream != nullptr) {

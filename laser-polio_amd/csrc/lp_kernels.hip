@@ -83,6 +83,12 @@ struct SpanLane {
   int32_t tile0, ntiles;
 };
 
+// Where a word of a node is (close_node): base + t * per_day + node * per_node, in words.
+struct CloseField {
+  uint32_t* base;
+  int32_t per_node, per_day;
+};
+
 struct Dev {
   // agent columns
   int8_t* state; int8_t* strain; int16_t* node_id;
@@ -106,7 +112,7 @@ struct Dev {
           *r_births, *r_deaths, *r_newexp, *r_newexp_bs, *r_riv, *r_rip, *r_ri_newexp_bs, *r_ipv,
           *r_siav, *r_siap, *r_sia_newexp_bs;
   // scratch
-  int32_t* day;   // [8] tick, end of the lp_run_days call, unused x2, the day record (today())
+  int32_t* day;   // [12] tick, end of the lp_run_days call, unused x2, the day record (today()), that of k_ei
   int32_t* stop_day; int32_t* err;
   const int4* spans; const int32_t* node_span_begin;
   const int32_t* tiles;    // every tile of every span: span << tpw_sh | tile of the span
@@ -135,6 +141,7 @@ struct Dev {
   uint32_t* sel_word;      // [sel_cap] round 1: a claimed agent's selection weight (all ones: recompute)
   int64_t* fin_prefix; int64_t* span_prefix;
   SpanLane* span_lane;     // [nodes][64]
+  const CloseField* close_tab;   // [2][64]
   int32_t* resv;           // [nodes] first list position of today's round-1 exposures (-1: appended)
   uint32_t* ticket;   // [4] last-block-done counters
   int64_t capacity; int32_t n_nodes, n_sims, K, nt, n_spans, tpw;
@@ -145,9 +152,13 @@ __device__ __forceinline__ bool sim_stopped(const Dev& d, int sim, int t) { retu
 
 // The current day's record at day + 4: {t, day_flags[t], ri_cnt[t], ri_cnt[t + 1]}, so
 // a kernel reads its day, flags and RI counts with one 16-byte load instead of a
-// load that depends on the day counter.  Written where the day is set (set_day)
-// and where it advances (k_day_end).
+// load that depends on the day counter.  k_ei, the first kernel of a list day, has a
+// copy of its own at day + 8: k_mix_foi moves that copy on while the day's kernels still
+// read day + 4, and the next k_ei (or k_advance, before a day without k_ei) brings
+// day + 4 up to it, so no kernel writes the record that it reads.  set_day and k_day_end
+// write both.
 __device__ __forceinline__ int4 today(const Dev& d) { return *reinterpret_cast<const int4*>(d.day + 4); }
+__device__ __forceinline__ int4 today_ei(const Dev& d) { return *reinterpret_cast<const int4*>(d.day + 8); }
 __device__ __forceinline__ int4 day_record(const Dev& d, int32_t t) {
   const int32_t f = t < d.nt ? d.day_flags[t] : 0;
   const int32_t r0 = t <= d.nt ? d.ri_cnt[t] : 0;          // ri_cnt has nt + 1 entries
@@ -157,7 +168,16 @@ __device__ __forceinline__ int4 day_record(const Dev& d, int32_t t) {
 __device__ __forceinline__ void set_today(const Dev& d, const int4& rec) {
   d.day[0] = rec.x;
   *reinterpret_cast<int4*>(d.day + 4) = rec;
+  *reinterpret_cast<int4*>(d.day + 8) = rec;
 }
+// A day begun by the k_finish before it: the other kernels' record and the empty list
+// of selected slots (one thread, before any of them).
+__device__ __forceinline__ void enter_day(const Dev& d, const int4& rec) {
+  d.day[0] = rec.x;
+  *reinterpret_cast<int4*>(d.day + 4) = rec;
+  d.sel_count[0] = 0;
+}
+__global__ void k_advance(Dev d) { enter_day(d, today_ei(d)); }
 
 __device__ __forceinline__ int32_t stage_day_flags(int32_t flags, int mask) {
   int32_t f = 0;
@@ -226,6 +246,25 @@ __device__ __forceinline__ DayBeginIn day_begin_load(const Dev& d, int n, int32_
   in.seg_end = d.seg_end[n];
   return in;
 }
+// Births of a VD step day: expected = step * rate * pop[t-1] in float64 as the reference
+// computes it (model.py:1712-1716), reproduced exactly in integer arithmetic; whole(b, f)
+// gets its integer part and fraction threshold.  `report`: the one thread that notes a
+// segment without room for all of them.
+template <typename Whole>
+__device__ __forceinline__ int64_t begin_births(const Dev& d, int32_t pop_prev, uint64_t rate, int32_t lnode, int32_t t,
+                                                uint64_t seed, int64_t live_end, int64_t seg_end, bool report,
+                                                Whole whole) {
+  uint64_t thr = 0;
+  int64_t b = pop_prev > 0 ? f64_mul_floor(rate, (uint32_t)pop_prev, &thr) : 0;
+  whole(b, thr);
+  if (thr) {
+    const uint4 o = philox(0u, (uint32_t)lnode, (uint32_t)t, ST_BIRTH, seed);
+    b += (uint64_t)o.x < thr ? 1 : 0;
+  }
+  const int64_t room = seg_end - live_end;
+  if (b > room) { b = room; if (report) atomicOr(d.err, ERR_CAPACITY); }
+  return b;
+}
 __device__ __forceinline__ void day_begin_apply(const Dev& d, int n, int32_t t, const DayBeginIn& in) {
   for (int k = 0; k < LP_MAX_STRAINS; ++k) d.newexp[n * LP_MAX_STRAINS + k] = 0;
   d.size[n] = 0; d.take_all[n] = 0; d.m_round[n] = 0;
@@ -234,18 +273,11 @@ __device__ __forceinline__ void day_begin_apply(const Dev& d, int n, int32_t t, 
   d.ei_cnt[(size_t)((t + 1) & 1) * d.n_nodes + n] = 0;
   if (in.stopped) return;
   if ((in.flags & LP_DAY_VD_STEP) && t >= 1) {
-    // expected = step * rate * pop[t-1] in float64 as the reference computes it
-    // (model.py:1712-1716), reproduced exactly in integer arithmetic
-    uint64_t thr = 0;
-    int64_t b = in.pop_prev > 0 ? f64_mul_floor(in.rate, (uint32_t)in.pop_prev, &thr) : 0;
-    d.birth_dbg[2 * n] = b;
-    d.birth_dbg[2 * n + 1] = (int64_t)thr;
-    if (thr) {
-      const uint4 o = philox(0u, (uint32_t)in.lnode, (uint32_t)t, ST_BIRTH, in.seed);
-      b += (uint64_t)o.x < thr ? 1 : 0;
-    }
-    const int64_t room = in.seg_end - in.live_end;
-    if (b > room) { b = room; atomicOr(d.err, ERR_CAPACITY); }
+    const int64_t b = begin_births(d, in.pop_prev, in.rate, in.lnode, t, in.seed, in.live_end, in.seg_end, true,
+                                   [&](int64_t whole, uint64_t f) {
+                                     d.birth_dbg[2 * n] = whole;
+                                     d.birth_dbg[2 * n + 1] = (int64_t)f;
+                                   });
     d.births[n] = (int32_t)b;
     d.live_end[n] = in.live_end + b;
   }
@@ -277,7 +309,7 @@ __device__ void day_stop_check(const Dev& d, int sim, int32_t t, int mask, int c
 }
 
 // Per node: births, per-day resets, early-stop rule.  Inside lp_run_days only the
-// first day launches it: k_day_end of each day begins the next one.
+// first day launches it: the end of each day (k_finish or k_day_end) begins the next one.
 __global__ void k_day_begin(Dev d, int mask, int32_t t, int32_t until) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n == 0) {
@@ -1074,7 +1106,8 @@ __device__ __forceinline__ int find_piece_node(const int32_t* off, int N, int32_
 __global__ void __launch_bounds__(WG) k_ei(Dev d, int mask) {
   // the piece offsets in LDS (when they fit) for the node lookup of each piece
   __shared__ int32_t s_off[EI_LDS_NODES + 1];
-  const int4 dy = today(d);
+  const int4 dy = today_ei(d);
+  if (blockIdx.x == 0 && threadIdx.x == 0) enter_day(d, dy);
   const int32_t t = dy.x;
   const int cur = t & 1, nxt = cur ^ 1;
   const int N = d.n_nodes, K = d.K;
@@ -2725,12 +2758,14 @@ __global__ void __launch_bounds__(WG) k_mix_foi(Dev d, int mask) {
   const int32_t t = dy.x;
   const int i0 = blockIdx.x * MIX_ROWS;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int4 next = blockIdx.x == 0 ? day_record(d, t + 1) : make_int4(0, 0, 0, 0);   // k_ei's
   if (!d.mix_buf) mix_rows(d, i0, part);
   const int i = i0 + w;
   const int32_t flags = stage_day_flags(dy.y, mask);
   // (wavefronts past the last node take it too, up to the barrier inside)
   mix_foi_node(d, i < d.n_nodes ? i : d.n_nodes - 1, d.ninfo[i < d.n_nodes ? i : d.n_nodes - 1], t, lane, w,
                !(flags & LP_DAY_TX), part, i < d.n_nodes);
+  if (blockIdx.x == 0 && threadIdx.x == 0) *reinterpret_cast<int4*>(d.day + 8) = next;
 }
 
 // One workgroup: plan sampling round `round` (probe offsets over nodes, list space).
@@ -3171,6 +3206,77 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
   }
 }
 
+// Per node: transmission incidence and the log rows of day t, in two parts as
+// day_begin: day_end_load (every input, the values the rows add to included, in flight
+// together) and day_end_apply (stores only).  ne, the day's exposures by strain, is the
+// caller's to fill in.
+struct DayEndIn {
+  int32_t sim, stop, flags, s_t, r_t, potp, pr;
+  int32_t ne[LP_MAX_STRAINS], ek[LP_MAX_STRAINS], ik[LP_MAX_STRAINS];
+  int32_t r_newexp, r_newexp_bs[LP_MAX_STRAINS], r_R;
+  int64_t carry_s, carry_spos;
+};
+__device__ __forceinline__ DayEndIn day_end_load(const Dev& d, int n, int32_t t, int32_t day_flags_t, int mask) {
+  DayEndIn in;
+  const int K = d.K;
+  const size_t row = (size_t)t * d.n_nodes + n;
+  const int64_t* tl = d.node_tally + (size_t)n * NPART;
+  in.sim = d.node_sim[n];
+  in.stop = d.stop_day[in.sim];
+  in.flags = stage_day_flags(day_flags_t, mask);
+#pragma unroll
+  for (int k = 0; k < LP_MAX_STRAINS; ++k) {
+    in.ne[k] = 0;
+    in.ek[k] = k < K ? (int32_t)tl[P_E0 + k] : 0;
+    in.ik[k] = k < K ? (int32_t)tl[P_I0 + k] : 0;
+    in.r_newexp_bs[k] = k < K ? d.r_newexp_bs[row * K + k] : 0;
+  }
+  in.s_t = (int32_t)tl[P_S];
+  in.r_t = (int32_t)tl[P_R];
+  in.potp = d.potp_run[n];
+  in.pr = d.p_run[n];
+  in.r_newexp = d.r_newexp[row];
+  in.r_R = d.r_R[row];
+  in.carry_s = d.node_carry[(size_t)n * 3 + 0];
+  in.carry_spos = d.node_carry[(size_t)n * 3 + 1];
+  return in;
+}
+__device__ __forceinline__ void day_end_apply(const Dev& d, int n, int32_t t, int mask, int tx_adjust,
+                                              const DayEndIn& in) {
+  const size_t N = d.n_nodes, row = (size_t)t * N + n;
+  const int K = d.K;
+  if (in.stop < t || !(in.flags & LP_DAY_TX)) return;
+  int32_t ne_tot = 0;
+#pragma unroll
+  for (int k = 0; k < LP_MAX_STRAINS; ++k) ne_tot += in.ne[k];
+  if ((mask & LP_STAGE_TRANSMISSION) && tx_adjust) {
+    d.r_newexp[row] = in.r_newexp + ne_tot;
+#pragma unroll
+    for (int k = 0; k < LP_MAX_STRAINS; ++k)
+      if (k < K) d.r_newexp_bs[row * K + k] = in.r_newexp_bs[k] + in.ne[k];
+    // every agent exposed by transmission left S and had a positive weight
+    d.node_carry[(size_t)n * 3 + 0] = in.carry_s - ne_tot;
+    d.node_carry[(size_t)n * 3 + 1] = in.carry_spos - ne_tot;
+  }
+  if (mask & LP_STAGE_LOG) {
+    int32_t e = 0, i = 0;
+#pragma unroll
+    for (int k = 0; k < LP_MAX_STRAINS; ++k) {
+      if (k >= K) break;
+      d.r_Ebs[row * K + k] = in.ek[k] + in.ne[k];
+      d.r_Ibs[row * K + k] = in.ik[k];
+      e += in.ek[k] + in.ne[k]; i += in.ik[k];
+    }
+    d.r_S[row] = in.s_t - ne_tot;
+    d.r_E[row] = e;
+    d.r_I[row] = i;
+    if (e + i > 0) d.sim_cases[in.sim] = 1;   // for the next day's early-stop rule
+    d.r_R[row] = in.r_R + in.r_t;
+    d.r_potp[row] = in.potp;
+    d.r_p[row] = in.pr;
+  }
+}
+
 // Per node: take-all nodes (size >= #positive-weight susceptibles) expose every
 // such agent; otherwise the node's later rounds (2, 3, ...) run here until
 // `size` distinct agents are exposed or no weight is left.  A round's probes are
@@ -3189,22 +3295,22 @@ __global__ void __launch_bounds__(WG) k_sample(Dev d) {
 // because k_sample's atomics on one node's counters serialised (14-node year 25.9 -> 23.4
 // ms without them).
 constexpr int FIN_LDS = 2048;
-template <int NT, int MINW>
-__global__ void __launch_bounds__(NT, MINW) k_finish(Dev d) {
-  const int4 dy = today(d);
-  const int32_t t = dy.x;
-  const int n = blockIdx.x;
+template <int NT>
+__device__ __forceinline__ void finish_node(const Dev& d, int32_t t, int n, int32_t* s_ne) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // the same in the wave's lanes
   __shared__ int64_t sh_base;
   __shared__ uint64_t s_sel[FIN_LDS];        // a round's selected entries when they fit
-  __shared__ int32_t s_ne[LP_MAX_STRAINS];   // the node's new exposures by strain (one global add each)
   __shared__ int32_t s_claimed;
   __shared__ int32_t s_cnt;                  // length of the node's list for tomorrow, which only this workgroup extends
   __shared__ int64_t s_spw[64];              // up to 64 spans: weight that left each span, not yet in its partial
   __shared__ int64_t s_w[64];                // and the weight each span has left
   const int32_t size = d.size[n], take_all = d.take_all[n], m1 = d.m_round[n];
-  if (size <= 0) return;
+  if (size <= 0) {
+    if (tid < LP_MAX_STRAINS) s_ne[tid] = 0;
+    __syncthreads();
+    return;
+  }
   const NodeInfo& ni = d.ninfo[n];
   const int nxt = (t + 1) & 1;
   const bool lane_spans = ni.n_spans <= 64;
@@ -3266,7 +3372,6 @@ __global__ void __launch_bounds__(NT, MINW) k_finish(Dev d) {
       if (lane_spans && tid < ni.n_spans && s_spw[tid] != 0)
         atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(ni.span_begin + tid) * NPART + P_SW),
                   (unsigned long long)s_spw[tid]);
-      if (tid < LP_MAX_STRAINS) d.newexp[n * LP_MAX_STRAINS + tid] = s_ne[tid];
       return;
     }
   }
@@ -3408,79 +3513,162 @@ __global__ void __launch_bounds__(NT, MINW) k_finish(Dev d) {
   if (lane_spans && tid < ni.n_spans && s_spw[tid] != 0)
     atomicAdd(reinterpret_cast<unsigned long long*>(d.partials + (size_t)(ni.span_begin + tid) * NPART + P_SW),
               (unsigned long long)s_spw[tid]);
-  if (tid < LP_MAX_STRAINS) d.newexp[n * LP_MAX_STRAINS + tid] = s_ne[tid];
   if (tid == 0 && s_cnt != cnt0) d.ei_cnt[(size_t)nxt * d.n_nodes + n] = s_cnt;
 }
 
-// Per node: transmission incidence and the log rows of day t, in two parts as
-// day_begin: day_end_load (every input, the values the rows add to included, in flight
-// together) and day_end_apply (stores only).
-struct DayEndIn {
-  int32_t sim, stop, flags, s_t, r_t, potp, pr;
-  int32_t ne[LP_MAX_STRAINS], ek[LP_MAX_STRAINS], ik[LP_MAX_STRAINS];
-  int32_t r_newexp, r_newexp_bs[LP_MAX_STRAINS], r_R;
-  int64_t carry_s, carry_spos;
-};
-__device__ __forceinline__ DayEndIn day_end_load(const Dev& d, int n, int32_t t, int32_t day_flags_t, int mask,
-                                                 int tx_adjust) {
-  DayEndIn in;
+// The end of a node's day and the beginning of its next one (day_end_apply, then
+// day_begin_apply) by one wavefront, for k_finish: every word they read and every word
+// they write has a lane, so k_finish has the reads on their way from its start in one
+// register and writes with one store.  A pass of its own (k_day_end) costs a list day 6 us
+// and a gap between kernels, two levels of loads of rows no longer in any cache; the whole
+// year with it / with its work by one thread at the end of k_finish / as here: 774 nodes
+// 33.5 / 32.2 / 31.4 ms, 14 nodes 22.9 / 22.0 / 21.4 ms, 64 replicates 69.7 / 67.8 / 67.2 ms,
+// 5000 nodes x 150 days 27.5 / 27.5 / 27.1 ms.  (One thread that loads from the start holds
+// forty registers and as many pointers, which the sampling rounds then spill.)
+enum : int { CL_S, CL_R, CL_POTP, CL_P, CL_NEWEXP, CL_RR, CL_POP, CL_E, CL_I = CL_E + LP_MAX_STRAINS,
+             CL_BS = CL_I + LP_MAX_STRAINS, CL_CS = CL_BS + LP_MAX_STRAINS, CL_CSPOS = CL_CS + 2,
+             CL_RATE = CL_CSPOS + 2, CL_LIVE = CL_RATE + 2, CL_SEG = CL_LIVE + 2, CL_SEED = CL_SEG + 2,
+             CL_SIM = CL_SEED + 2, CL_LNODE, CL_N };
+// written: the day's end (to CO_CASES), the next day's beginning (to CO_CNT), its births
+enum : int { CO_NEWEXP, CO_S, CO_E, CO_I, CO_R, CO_POTP, CO_P, CO_CS, CO_CSPOS = CO_CS + 2, CO_BS = CO_CSPOS + 2,
+             CO_EBS = CO_BS + LP_MAX_STRAINS, CO_IBS = CO_EBS + LP_MAX_STRAINS, CO_CASES = CO_IBS + LP_MAX_STRAINS,
+             CO_NE, CO_SIZE = CO_NE + LP_MAX_STRAINS, CO_TAKE, CO_M, CO_BIRTHS, CO_NB, CO_CNT = CO_NB + 2,
+             CO_DBG, CO_LIVE = CO_DBG + 4, CO_N = CO_LIVE + 2 };
+static_assert(CL_N <= 64 && CO_N <= 64, "one word per lane");
+// Dev::close_tab: the words read, then the words written
+inline void close_fields(const Dev& d, CloseField* tab) {
+  const int32_t N = d.n_nodes;
+  for (int l = 0; l < 128; ++l) tab[l] = {reinterpret_cast<uint32_t*>(d.node_tally), 0, 0};   // unused lanes
+  auto put = [&](int l, const void* base, size_t node_bytes, int32_t per_day, int words) {
+    for (int j = 0; j < words; ++j)
+      tab[l + j] = {reinterpret_cast<uint32_t*>(const_cast<void*>(base)) + j, (int32_t)(node_bytes / 4), per_day};
+  };
+  put(CL_S, d.node_tally + P_S, NPART * 8, 0, 1);
+  put(CL_R, d.node_tally + P_R, NPART * 8, 0, 1);
+  put(CL_POTP, d.potp_run, 4, 0, 1);
+  put(CL_P, d.p_run, 4, 0, 1);
+  put(CL_NEWEXP, d.r_newexp, 4, N, 1);
+  put(CL_RR, d.r_R, 4, N, 1);
+  put(CL_POP, d.r_pop, 4, N, 1);
+  put(CL_CS, d.node_carry, 24, 0, 2);
+  put(CL_CSPOS, d.node_carry + 1, 24, 0, 2);
+  put(CL_RATE, d.birth_rate_step, 8, 0, 2);
+  put(CL_LIVE, d.live_end, 8, 0, 2);
+  put(CL_SEG, d.seg_end, 8, 0, 2);
+  put(CL_SEED, &d.ninfo->seed, sizeof(NodeInfo), 0, 2);
+  put(CL_SIM, &d.ninfo->sim, sizeof(NodeInfo), 0, 1);
+  put(CL_LNODE, &d.ninfo->lnode, sizeof(NodeInfo), 0, 1);
+  CloseField* in = tab;
+  tab += 64;
+  put(CO_NEWEXP, d.r_newexp, 4, N, 1);
+  put(CO_S, d.r_S, 4, N, 1);
+  put(CO_E, d.r_E, 4, N, 1);
+  put(CO_I, d.r_I, 4, N, 1);
+  put(CO_R, d.r_R, 4, N, 1);
+  put(CO_POTP, d.r_potp, 4, N, 1);
+  put(CO_P, d.r_p, 4, N, 1);
+  put(CO_CS, d.node_carry, 24, 0, 2);
+  put(CO_CSPOS, d.node_carry + 1, 24, 0, 2);
+  put(CO_CASES, d.sim_cases, 4, 0, 1);   // of the node's simulation
+  put(CO_SIZE, d.size, 4, 0, 1);
+  put(CO_TAKE, d.take_all, 4, 0, 1);
+  put(CO_M, d.m_round, 4, 0, 1);
+  put(CO_BIRTHS, d.births, 4, 0, 1);
+  put(CO_NB, d.nb_begin, 8, 0, 2);
+  put(CO_CNT, d.ei_cnt, 4, N, 1);        // per_day: of the tick's parity
+  put(CO_DBG, d.birth_dbg, 16, 0, 4);
+  put(CO_LIVE, d.live_end, 8, 0, 2);
+  for (int k = 0; k < LP_MAX_STRAINS; ++k) put(CO_NE + k, d.newexp + k, 4 * LP_MAX_STRAINS, 0, 1);
+  for (int k = 0; k < d.K; ++k) {
+    put(CO_BS + k, d.r_newexp_bs + k, 4 * (size_t)d.K, N * d.K, 1);
+    put(CO_EBS + k, d.r_Ebs + k, 4 * (size_t)d.K, N * d.K, 1);
+    put(CO_IBS + k, d.r_Ibs + k, 4 * (size_t)d.K, N * d.K, 1);
+    in[CL_E + k] = {reinterpret_cast<uint32_t*>(d.node_tally + P_E0 + k), NPART * 2, 0};
+    in[CL_I + k] = {reinterpret_cast<uint32_t*>(d.node_tally + P_I0 + k), NPART * 2, 0};
+    in[CL_BS + k] = {reinterpret_cast<uint32_t*>(d.r_newexp_bs + k), d.K, N * d.K};
+  }
+}
+// v: word `lane` as read; stop: the simulation's stop day; ne: today's exposures by strain
+__device__ __forceinline__ void close_node(const Dev& d, int n, int32_t t, int lane, uint32_t v, int32_t stop,
+                                           int32_t flags_t, int32_t flags_next, int32_t until, const int32_t* ne) {
+  const CloseField cf = d.close_tab[64 + lane];
+  auto w = [&](int l) { return (int32_t)__builtin_amdgcn_readlane((int)v, l); };
+  auto w64 = [&](int l) { return (int64_t)(((uint64_t)(uint32_t)w(l + 1) << 32) | (uint32_t)w(l)); };
   const int K = d.K;
-  const size_t row = (size_t)t * d.n_nodes + n;
-  const int64_t* tl = d.node_tally + (size_t)n * NPART;
-  in.sim = d.node_sim[n];
-  in.stop = d.stop_day[in.sim];
-  in.flags = stage_day_flags(day_flags_t, mask);
+  const int32_t sim = w(CL_SIM);
+  uint32_t out = 0;     // what lane `lane` writes (0: the counters a day starts from)
+  auto set = [&](int l, int32_t x) { out = lane == l ? (uint32_t)x : out; };
+  auto set64 = [&](int l, int64_t x) { set(l, (int32_t)x); set(l + 1, (int32_t)(x >> 32)); };
+  // the day's end
+  int32_t ne_tot = 0, e = 0, i = 0;
 #pragma unroll
   for (int k = 0; k < LP_MAX_STRAINS; ++k) {
-    in.ne[k] = (tx_adjust && k < K) ? d.newexp[n * LP_MAX_STRAINS + k] : 0;
-    in.ek[k] = k < K ? (int32_t)tl[P_E0 + k] : 0;
-    in.ik[k] = k < K ? (int32_t)tl[P_I0 + k] : 0;
-    in.r_newexp_bs[k] = k < K ? d.r_newexp_bs[row * K + k] : 0;
+    if (k >= K) break;
+    ne_tot += ne[k];
+    e += w(CL_E + k) + ne[k];
+    i += w(CL_I + k);
+    set(CO_BS + k, w(CL_BS + k) + ne[k]);
+    set(CO_EBS + k, w(CL_E + k) + ne[k]);
+    set(CO_IBS + k, w(CL_I + k));
   }
-  in.s_t = (int32_t)tl[P_S];
-  in.r_t = (int32_t)tl[P_R];
-  in.potp = d.potp_run[n];
-  in.pr = d.p_run[n];
-  in.r_newexp = d.r_newexp[row];
-  in.r_R = d.r_R[row];
-  in.carry_s = d.node_carry[(size_t)n * 3 + 0];
-  in.carry_spos = d.node_carry[(size_t)n * 3 + 1];
-  return in;
-}
-__device__ __forceinline__ void day_end_apply(const Dev& d, int n, int32_t t, int mask, int tx_adjust,
-                                              const DayEndIn& in) {
-  const size_t N = d.n_nodes, row = (size_t)t * N + n;
-  const int K = d.K;
-  if (in.stop < t || !(in.flags & LP_DAY_TX)) return;
-  int32_t ne_tot = 0;
-#pragma unroll
-  for (int k = 0; k < LP_MAX_STRAINS; ++k) ne_tot += in.ne[k];
-  if ((mask & LP_STAGE_TRANSMISSION) && tx_adjust) {
-    d.r_newexp[row] = in.r_newexp + ne_tot;
-#pragma unroll
-    for (int k = 0; k < LP_MAX_STRAINS; ++k)
-      if (k < K) d.r_newexp_bs[row * K + k] = in.r_newexp_bs[k] + in.ne[k];
-    // every agent exposed by transmission left S and had a positive weight
-    d.node_carry[(size_t)n * 3 + 0] = in.carry_s - ne_tot;
-    d.node_carry[(size_t)n * 3 + 1] = in.carry_spos - ne_tot;
+  set(CO_NEWEXP, w(CL_NEWEXP) + ne_tot);
+  set(CO_S, w(CL_S) - ne_tot);
+  set(CO_E, e);
+  set(CO_I, i);
+  set(CO_R, w(CL_RR) + w(CL_R));
+  set(CO_POTP, w(CL_POTP));
+  set(CO_P, w(CL_P));
+  set64(CO_CS, w64(CL_CS) - ne_tot);
+  set64(CO_CSPOS, w64(CL_CSPOS) - ne_tot);
+  set(CO_CASES, 1);
+  bool on = false;
+  if (stop >= t && (stage_day_flags(flags_t, LP_STAGE_ALL) & LP_DAY_TX)) {
+    const int lk = lane - CO_BS;   // the rows by strain have K of LP_MAX_STRAINS
+    on = lane < CO_BS || (lane < CO_CASES && lk % LP_MAX_STRAINS < K) || (lane == CO_CASES && e + i > 0);
   }
-  if (mask & LP_STAGE_LOG) {
-    int32_t e = 0, i = 0;
-#pragma unroll
-    for (int k = 0; k < LP_MAX_STRAINS; ++k) {
-      if (k >= K) break;
-      d.r_Ebs[row * K + k] = in.ek[k] + in.ne[k];
-      d.r_Ibs[row * K + k] = in.ik[k];
-      e += in.ek[k] + in.ne[k]; i += in.ik[k];
+  // the next day's beginning
+  if (t + 1 < until) {
+    const int64_t live = w64(CL_LIVE);
+    set64(CO_NB, live);
+    on = on || (lane > CO_CASES && lane <= CO_CNT);
+    if (stop >= t + 1 && (stage_day_flags(flags_next, LP_STAGE_ALL) & LP_DAY_VD_STEP)) {
+      const int64_t b = begin_births(d, w(CL_POP), (uint64_t)w64(CL_RATE), w(CL_LNODE), t + 1,
+                                     (uint64_t)w64(CL_SEED), live, w64(CL_SEG), lane == 0,
+                                     [&](int64_t whole, uint64_t f) {
+                                       set64(CO_DBG, whole);
+                                       set64(CO_DBG + 2, (int64_t)f);
+                                     });
+      set(CO_BIRTHS, (int32_t)b);
+      set64(CO_LIVE, live + b);
+      on = on || (lane > CO_CNT && lane < CO_N);
     }
-    d.r_S[row] = in.s_t - ne_tot;
-    d.r_E[row] = e;
-    d.r_I[row] = i;
-    if (e + i > 0) d.sim_cases[in.sim] = 1;   // for the next day's early-stop rule
-    d.r_R[row] = in.r_R + in.r_t;
-    d.r_potp[row] = in.potp;
-    d.r_p[row] = in.pr;
   }
+  const int32_t at = lane == CO_CNT ? t & 1 : t, of = lane == CO_CASES ? sim : n;
+  if (on) cf.base[(int64_t)at * cf.per_day + (int64_t)of * cf.per_node] = out;
+}
+
+// finish_node, then with `end` the end of the node's day (close_node) by the last
+// wavefront, the one with the least to do in a round of few probes.
+template <int NT, int MINW>
+__global__ void __launch_bounds__(NT, MINW) k_finish(Dev d, int end) {
+  __shared__ int32_t s_ne[LP_MAX_STRAINS];   // the node's new exposures by strain
+  const int4 dy = today(d);
+  const int32_t t = dy.x;
+  const int n = blockIdx.x;
+  const int lane = threadIdx.x & 63;
+  const bool closes = end && __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) == NT / 64 - 1;
+  uint32_t v = 0;
+  int32_t stop = 0, flags_next = 0, until = 0;
+  if (closes) {
+    const CloseField cf = d.close_tab[lane];
+    v = cf.base[(int64_t)t * cf.per_day + (int64_t)n * cf.per_node];
+    stop = d.stop_day[d.node_sim[n]];
+    flags_next = d.day[9];   // of k_ei's record, moved on by k_mix_foi
+    until = d.day[1];
+  }
+  finish_node<NT>(d, t, n, s_ne);
+  if (!end && threadIdx.x < LP_MAX_STRAINS) d.newexp[n * LP_MAX_STRAINS + threadIdx.x] = s_ne[threadIdx.x];
+  if (closes) close_node(d, n, t, lane, v, stop, dy.y, flags_next, until, s_ne);
 }
 
 // ei_piece_off = exclusive prefix over nodes of the pieces of list b (the last
@@ -3494,11 +3682,10 @@ __device__ void ei_plan(const Dev& d, int b) {
   if (threadIdx.x == 0) d.ei_piece_off[N] = (int32_t)total;
 }
 
-// Per node: transmission incidence and the log rows.  With `advance`: when the
-// next tick is inside the current lp_run_days call (before day[1]), each node's
-// thread also begins that day (day_begin_node) and the last workgroup runs the
-// early-stop rule for it; the last workgroup plans the next day's E / I list
-// pieces and moves the day counter.
+// Per node: transmission incidence and the log rows of a day outside the list kinds
+// (k_finish ends those).  With `advance`: when the next tick is inside the current
+// lp_run_days call (before day[1]), each node's thread also begins that day
+// (day_begin_apply), and the last workgroup moves the day counter.
 __global__ void __launch_bounds__(WG) k_day_end(Dev d, int mask, int tx_adjust, int advance) {
   const int4 dy = today(d);
   const int32_t t = dy.x;
@@ -3509,7 +3696,10 @@ __global__ void __launch_bounds__(WG) k_day_end(Dev d, int mask, int tx_adjust, 
   if (n < d.n_nodes) {
     // the next day's inputs are loaded before today's log rows are stored
     // every input of the day's end and of the next day's beginning loads before any store
-    const DayEndIn ein = day_end_load(d, n, t, dy.y, mask, tx_adjust);
+    DayEndIn ein = day_end_load(d, n, t, dy.y, mask);
+#pragma unroll
+    for (int k = 0; k < LP_MAX_STRAINS; ++k)
+      ein.ne[k] = (tx_adjust && k < d.K) ? d.newexp[n * LP_MAX_STRAINS + k] : 0;
     const DayBeginIn in = begin_next ? day_begin_load(d, n, t + 1, mask) : DayBeginIn{};
     day_end_apply(d, n, t, mask, tx_adjust, ein);
     if (begin_next) day_begin_apply(d, n, t + 1, in);
@@ -3535,7 +3725,7 @@ __global__ void __launch_bounds__(WG) k_day_end(Dev d, int mask, int tx_adjust, 
 
 // The piece plan of today's E / I list for k_ei when the node count exceeds what its
 // workgroups scan into LDS themselves (one workgroup).
-__global__ void __launch_bounds__(WG) k_ei_plan(Dev d) { ei_plan(d, today(d).x & 1); }
+__global__ void __launch_bounds__(WG) k_ei_plan(Dev d) { ei_plan(d, today_ei(d).x & 1); }
 
 
 }  // namespace lp
