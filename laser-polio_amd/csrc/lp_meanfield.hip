@@ -52,8 +52,9 @@ __device__ __forceinline__ void lds_barrier() {
 // us for either, one workgroup of 23 nodes 0.36 and 0.53 us (a launch per day: about 6 and 11).
 // The network's adjoint N_bar[j][i] += beta_j (mbar_i - mbar_j) of all days is summed
 // by one pass afterwards (k_mf_net_bar) instead of read and written once a day.
-// In the adjoint, h_i = g_bar_i r0_i / pop_i of a day goes to its season_part row first:
-// mbar_i = h_i season_t is what the network sees, and season_part_i = h_i m_i at the end.
+// In the adjoint, mbar_i = ((g_bar_i season_t) r0_i) / pop_i of a day goes to its season_part
+// row first (h below; see day_adjoint): the network sees it there, and at the end
+// season_part_i = mbar_i / season_t m_i takes its place.
 
 // x plus the other lanes' of its row of 16, in every lane of the row.
 template <int N>
@@ -99,7 +100,14 @@ __device__ __forceinline__ DayOut day_forward(const lp_mf_model& m, const Node& 
 }
 
 // The elementwise part of a day's adjoint: from the adjoints of the state after the day,
-// updates aS and aE to the day's start, adds to r0_bar, returns h (see above).
+// updates aS and aE to the day's start, adds to r0_bar, returns the day's row entry: mbar, the
+// adjoint of the mixed weight, whose rounding every node and day shares through the network
+// (((g_bar r0) inv_pop) season in its place, the same product in another order, moved the
+// gradients of E and I by 1e-6 of their size, away from float64 on some inputs: 2.6e-6 for
+// 1.9e-6).  season_part is mbar / season times m; a season so small that the quotient could
+// be lost keeps the row without its factor.
+__device__ __forceinline__ bool row_has_season(float season) { return fabsf(season) >= 0x1p-20f; }
+__device__ __forceinline__ float row_scale(float season) { return row_has_season(season) ? 1.0f : season; }   // mbar / row
 __device__ __forceinline__ float day_adjoint(const lp_mf_model& m, const Node& c, float season, float S0, float mm,
                                              float g, float ainc, float& aS, float& aE, float aI, float& r0_bar) {
   const float p = -lp::expm1f_lp(-g);
@@ -109,7 +117,7 @@ __device__ __forceinline__ float day_adjoint(const lp_mf_model& m, const Node& c
   r0_bar += ((g_bar * mm) * season) * c.inv_pop;
   aS = aS + (lam_bar * c.rho) * p;
   aE = aE * (1.0f - m.inv_tau_e) + aI * m.inv_tau_e;
-  return (g_bar * c.r0) * c.inv_pop;
+  return ((row_has_season(season) ? g_bar * season : g_bar) * c.r0) * c.inv_pop;
 }
 // aI at the day's start from aI after it and s = sum_i N_ji mbar_i.
 __device__ __forceinline__ float adjoint_i(const lp_mf_model& m, const Node& c, float aI, float mbar, float s) {
@@ -262,7 +270,7 @@ __global__ void __launch_bounds__(1024) k_mf_adj_wg(lp_mf_model m, int t0, int d
       float mbar = 0.0f;
       if (own) {
         const float hd = day_adjoint(m, c, season, in.S0[u], in.mm[u], in.g[u], in.ainc[u], s, e, x, r0);
-        mbar = hd * season;
+        mbar = hd * row_scale(season);
         v[d & 1][i] = mbar;
         h[(size_t)d * n + i] = hd;
       }
@@ -442,9 +450,9 @@ __global__ void __launch_bounds__(RES_WG) k_mf_adj_res(lp_mf_model m, int t0, in
       if (own) {
         const float hd = day_adjoint(m, c, season, in.S0[u], in.mm[u], in.g[u], in.ainc[u], s, e, x, r0);
         publish(h + (size_t)d * n + i, hd);
-        mbar = hd * season;
+        mbar = hd * row_scale(season);
       }
-      if (!await_row<K>(h + (size_t)d * n, n, season, v[d & 1], &s_late)) return;
+      if (!await_row<K>(h + (size_t)d * n, n, row_scale(season), v[d & 1], &s_late)) return;
       const float sum = rows.apply(v[d & 1], lane);
       if (own) x = adjoint_i(m, c, x, mbar, sum);
       if ((d & 63) == 0 && d > 0) seasons.load(m.season, t0, days, d - 1);
@@ -520,7 +528,7 @@ __global__ void __launch_bounds__(WG) k_mf_adj_day(lp_mf_model m, int t0, int da
   aE[j] = e;
   r0_bar[j] = r0;
   h[r] = hj;
-  mb_out[j] = hj * season;
+  mb_out[j] = hj * row_scale(season);
 }
 
 // ---- after the days --------------------------------------------------------------------
@@ -552,7 +560,7 @@ __global__ void __launch_bounds__(WG) k_mf_net_bar(lp_mf_model m, int t0, int da
     for (int a = 0; a < PER; ++a) {
       const int day = lo + q + a * (WG / NB_TILE);
       const size_t r = (size_t)(day < hi ? day : hi - 1) * n;
-      season[a] = m.season[t0 + (day < hi ? day : hi - 1)];
+      season[a] = row_scale(m.season[t0 + (day < hi ? day : hi - 1)]);
       x[a] = h[r + ci];
       y[a] = h[r + cj];
       b[a] = I[r + cj];
@@ -581,9 +589,15 @@ __global__ void __launch_bounds__(WG) k_mf_net_bar(lp_mf_model m, int t0, int da
   }
 }
 
-// season_part = h m, in place.
-__global__ void __launch_bounds__(WG) k_mf_season(float* h, const float* msave, int64_t n) {
-  for (int64_t j = (int64_t)blockIdx.x * WG + threadIdx.x; j < n; j += (int64_t)gridDim.x * WG) h[j] = h[j] * msave[j];
+// season_part from the rows, in place.
+__global__ void __launch_bounds__(WG) k_mf_season(lp_mf_model m, int t0, int days, float* h, const float* msave) {
+  const int i = blockIdx.x * WG + threadIdx.x;
+  if (i >= m.n) return;
+  for (int d = blockIdx.y; d < days; d += gridDim.y) {
+    const float season = m.season[t0 + d], mm = msave[(size_t)d * m.n + i];
+    float* p = h + (size_t)d * m.n + i;
+    *p = (row_has_season(season) ? *p / season : *p) * mm;
+  }
 }
 
 // Which way a call goes.  The one-workgroup kernels lead the resident ones up to the 256
@@ -715,7 +729,8 @@ int lp_mf_adjoint_days(const lp_mf_model* model, int32_t t0, int32_t t1, const f
   }
   const int tiles = (n + lp_mf::NB_TILE - 1) / lp_mf::NB_TILE;
   hipLaunchKernelGGL(lp_mf::k_mf_net_bar, dim3(tiles, tiles), dim3(lp_mf::WG), 0, s, m, t0, days, I, h, net_bar);
-  hipLaunchKernelGGL(lp_mf::k_mf_season, dim3(lp_mf::fill_grid(cells)), dim3(lp_mf::WG), 0, s, h, m_save, cells);
+  hipLaunchKernelGGL(lp_mf::k_mf_season, dim3((n + lp_mf::WG - 1) / lp_mf::WG, std::min(days, 1024)), dim3(lp_mf::WG), 0, s, m, t0,
+                     days, h, m_save);
   return hipGetLastError() == hipSuccess ? LP_OK : LP_ERR_HIP;
 }
 
