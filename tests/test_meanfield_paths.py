@@ -91,3 +91,28 @@ def test_rollout_under_graph_capture(n):
             torch.cuda.synchronize()
             err = float((out - eager).norm() / eager.norm())
             assert err <= 16 * 11 * 2.0**-24, (k, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [40, 300, 2100])
+def test_days_of_no_or_little_season_match_float64(n):
+    """A day's row keeps the season as a factor unless it is below 2^-20: both sides of that
+    line, zero and a season of the other sign."""
+    print(f"[meanfield] season edges n={n}", flush=True)
+    edges = [0.0, 1.0, 2.0**-19, 2.0**-20, 2.0**-21, 0.0, -0.25, 1.5, 1e-12, 1.0]
+    T = len(edges)
+    x = _inputs(n, T)
+    x[2] = torch.tensor(edges, dtype=torch.float32, device="cuda")
+    got = _run(adj.rollout, x, torch.float32)
+    x[2] = x[2][:, None].expand(T, n).contiguous()
+    want = _run(adj.rollout_reference, x, torch.float64)
+    terms = want[3]
+    want[3] = terms.sum(dim=1)
+    tol = 2 * 8 * (T + 2) * 2.0**-24      # as in test_every_path_matches_float64
+    off = ~torch.eye(n, dtype=torch.bool, device="cuda")
+    for name, a, b in zip(("inc", "r0s", "net", "season", "S", "E", "I"), got, want):
+        a = a.double()
+        if name == "net":
+            a, b = a[off], b[off]
+        size = terms.abs().sum(dim=1) if name == "season" else b
+        assert float((a - b).norm() / size.norm().clamp_min(1e-30)) <= tol, name
