@@ -231,9 +231,10 @@ def dense_model_bytes(res, flags, t0, t1):
 
 def _rocprof_days(path, value=False):
     """Rows of a rocprofv3 CSV (kernel trace, or counter collection with one counter) in
-    dispatch order, each with the simulated tick it belongs to: the dispatches up to and
-    including the t-th k_day_end make up tick t.  Returns [(tick, kernel name, ns or
-    counter value)]; counter rows of one dispatch are summed."""
+    dispatch order, each with the simulated tick it belongs to: a tick ends with its
+    k_day_end, or with a k_finish that no k_day_end follows (days from the E / I list).
+    Returns [(tick, kernel name, ns or counter value)]; counter rows of one dispatch are
+    summed."""
     import csv
 
     per = {}
@@ -249,10 +250,11 @@ def _rocprof_days(path, value=False):
             else:
                 per[k] = [r["Kernel_Name"], v]
     out, tick = [], 0
-    for k in sorted(per):
-        name, v = per[k]
+    rows = [per[k] for k in sorted(per)]
+    for i, (name, v) in enumerate(rows):
         out.append((tick, name, v))
-        if "k_day_end" in name:
+        follows = rows[i + 1][0] if i + 1 < len(rows) else ""
+        if "k_day_end" in name or ("k_finish" in name and "k_day_end" not in follows):
             tick += 1
     return out
 

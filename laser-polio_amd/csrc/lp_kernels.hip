@@ -24,16 +24,16 @@
 //                  weighted sampling without replacement by rounds of with-
 //                  replacement probes + unique (model.py:1089-1122): every probe
 //                  searches its node's span prefix, then a span's chunks, then one
-//                  chunk, one wavefront per probe; round 1 grid-wide (planned
+//                  chunk, four probes per wavefront; round 1 grid-wide (planned
 //                  inside k_sample, by k_plan above 8191 nodes; k_sample claims
 //                  its agents, k_finish makes them E), later rounds and the
 //                  take-all nodes per node in k_finish; each exposed agent's strain is drawn
 //                  as it is exposed (S -> E) and it joins the next day's E / I list
 //                                                               model.py:1125-1147
-//   k_day_end      per node: log rows + transmission incidence; its last
-//                  workgroup plans the next day's list pieces and advances the day
-//                  counter                             model.py:1436-1441, 1461-1483
-// A day is replayed as one hipGraph (one graph per day kind).
+//   k_day_end      per node: log rows + transmission incidence of tick 0, dense days and
+//                  stage calls; on list days the end of k_finish does it
+//                                                       model.py:1436-1441, 1461-1483
+// Days are replayed as hipGraphs (per day kind, runs of 1, 2, 4 or 8 days).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <limits.h>
@@ -286,8 +286,8 @@ __device__ void day_begin_node(const Dev& d, int n, int32_t t, int mask) {
   day_begin_apply(d, n, t, day_begin_load(d, n, t, mask));
 }
 
-// sim_cases[sim]: 1 when a node of the sim logged E or I on the previous day (set by
-// k_day_end), 0 when none did; CASES_CHECKED when today's early-stop rule has run
+// sim_cases[sim]: 1 when a node of the sim logged E or I on the previous day (set by the
+// day's end), 0 when none did; CASES_CHECKED when today's early-stop rule has run
 // already (k_day_begin, which sums the rows).  k_node_reduce runs the rule for
 // days begun inside lp_run_days and clears the flag for today's log.
 constexpr int32_t CASES_CHECKED = 2;
