@@ -117,6 +117,7 @@ struct lp_ctx {
   bool rec_dirty = false;                          // agent records newer than the bound columns
   bool rec_actual = true;                          // records hold the actual timers of E / I agents
   bool ran = false;                                // a day or stage has been queued
+  int32_t ri_done = -1;                            // latest tick whose RI step, if it has one, has been queued
   std::vector<int32_t> day_flags_h;
   std::vector<int32_t> ri_cnt_h;
   std::string err;
@@ -289,13 +290,15 @@ bool same_list_kind(const lp_ctx* c, int32_t a, int32_t b, int kind) {
 
 // Everything carried from day to day rebuilt from the bound columns, for tick t (the day
 // set by it, `until` as for enqueue_day); with `lists` the E / I list of tick t too; ri: the
-// stages to run include today's RI step.
+// stages to run include today's RI step.  A stage call may recount after today's RI: the RI
+// candidates are then those of the next RI day.
 void enqueue_recount(lp_ctx* c, int32_t t, int32_t until, bool lists, bool ri) {
   const int n = std::max(c->cfg.n_nodes, c->n_spans);
   if (c->rec_dirty) enqueue_sync_columns(c);   // the pass reads the columns
   hipLaunchKernelGGL(lp::k_recount_begin, dim3(grid_of(n, lp::WG)), dim3(lp::WG), 0, c->stream, c->d, ri ? 1 : 0,
                      t, until);
-  hipLaunchKernelGGL(lp::k_recount, dim3(c->n_tiles), dim3(lp::WG), 0, c->stream, c->d, lists ? 1 : 0);
+  hipLaunchKernelGGL(lp::k_recount, dim3(c->n_tiles), dim3(lp::WG), 0, c->stream, c->d, lists ? 1 : 0,
+                     !ri && c->ri_done == t ? 1 : 0);
   c->recount_pending = false;
   c->rec_dirty = true;
   c->rec_actual = true;
@@ -636,6 +639,7 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
   int32_t t = t_begin;
   if (t == 0) {
     // tick 0 only logs; the tally of its dense pass lists the E / I agents for tick 1
+    c->ri_done = 0;
     enqueue_recount(c, t, t_end, false, false);
     if ((rc = enqueue_day(c, t, lp::KIND_PLAIN, LP_STAGE_LOG, 0, true, first, t_end))) return rc;
     first = false;
@@ -684,6 +688,7 @@ int lp_run_days(lp_ctx* c, int32_t t_begin, int32_t t_end, int32_t use_graph) {
     }
     first = false;
   }
+  c->ri_done = t_end - 1;
   return LP_OK;
 }
 
@@ -695,7 +700,9 @@ int lp_step_stage(lp_ctx* c, int32_t t, int32_t mask) {
   first_run(c, t);
   const bool fused_tx_log = (mask & LP_STAGE_TRANSMISSION) && (mask & LP_STAGE_LOG);
   enqueue_actualize(c);
-  if (c->recount_pending) enqueue_recount(c, t, 0, false, host_stage_flags(c->day_flags_h[t], mask) & LP_DAY_RI);
+  const bool ri = host_stage_flags(c->day_flags_h[t], mask) & LP_DAY_RI;
+  if (c->recount_pending) enqueue_recount(c, t, 0, false, ri);
+  if (ri) c->ri_done = t;
   c->list_tick = -1;   // stage calls do not keep the E / I list
   return enqueue_day(c, t, day_kind(c, t, mask), mask, fused_tx_log || !(mask & LP_STAGE_LOG) ? 1 : 0, false, true);
 }

@@ -770,13 +770,14 @@ __global__ void __launch_bounds__(WG) k_recount_begin(Dev d, int ri, int32_t t, 
 // One workgroup per tile, one quad of slots per thread: the agent records from the columns; per chunk the weight of its S agents and
 // the earliest death date of its live ones; per span its weight; per node #S, #S with
 // positive weight, #R, the potentially paralysed and the paralysed; with `lists` the node's
-// E / I list of today (timers as of the start of today); the RI candidates of the next RI
-// day (today's, if today is one: live agents, not chronically missed, whose window can
-// still open).  Bound by HBM: 28 bytes read and 16 written per slot, every load of a
+// E / I list of today (timers as of the start of today); the RI candidates (live agents, not
+// chronically missed, whose window can still open) of the RI day ahead: today, if it is one,
+// or, with `ri_done` (today's RI has run: a stage call later in the day), the next one, each
+// in the buffer that its pass will read.  Bound by HBM: 28 bytes read and 16 written per slot, every load of a
 // thread in flight at once: 2.45 ms at 269 M slots, 4.8 TB/s, what a large copy reaches.
 // (A pass per span that also ran the day took 2.7 ms there and a separate record pass
 // 3.2 ms; at 5.4 M slots, 330 workgroups of 16 tiles each, 280 and 50 us against 61 us.)
-__global__ void __launch_bounds__(WG) k_recount(Dev d, int lists) {
+__global__ void __launch_bounds__(WG) k_recount(Dev d, int lists, int ri_done) {
   const int tile = d.tiles[blockIdx.x], u = tile & ((1 << d.tpw_sh) - 1);
   const int4 span = d.spans[tile >> d.tpw_sh];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -840,7 +841,8 @@ __global__ void __launch_bounds__(WG) k_recount(Dev d, int lists) {
   // wavefront's own atomics on one node's list lengths serialised: 214 us for 5.4 M slots
   // of 14 nodes whose every agent was an RI candidate).  Without an RI day ahead no
   // candidates are listed.
-  const bool ri_ahead = d.ri_cnt[d.nt] > dy.z;
+  const int32_t ri_before = ri_done ? dy.w : dy.z;        // RI days before the one ahead
+  const bool ri_ahead = d.ri_cnt[d.nt] > ri_before;
   if (!lists) ei = 0;
   if (!ri_ahead) cand = 0;
   const int32_t mine = __popc(ei) | (__popc(cand) << 16);  // at most 256 of each in a wave
@@ -850,7 +852,7 @@ __global__ void __launch_bounds__(WG) k_recount(Dev d, int lists) {
   __shared__ int32_t s_l[WG / 64], s_base[2];
   if (lane == 63) { s_w[wave] = cw; s_n[wave] = c_n; s_p[wave] = c_p; s_l[wave] = incl; }
   __syncthreads();
-  const int b = dy.z & 1;
+  const int b = ri_before & 1;
   if (tid < 8) {
     int64_t v = 0;
 #pragma unroll
