@@ -316,7 +316,10 @@ int enqueue_day(lp_ctx* c, int32_t t, int kind, int mask, int tx_adjust, bool ad
   // passes that read the records need their actual timers (never inside a captured
   // graph: run_days calls enqueue_actualize before capturing)
   if (!list_kind(kind)) enqueue_actualize(c);
-  if (begin) hipLaunchKernelGGL(lp::k_day_begin, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask, t, until);
+  if (begin) {
+    const int relist = !list_kind(kind) && (kind & lp::FULL_RI) ? 1 : 0;   // k_full lists every RI candidate
+    hipLaunchKernelGGL(lp::k_day_begin, dim3(grid_of(N, 256)), dim3(256), 0, s, d, mask, t, until, relist);
+  }
   const bool ev = c->timing;
   if (ev) {
     if (c->ev_used + 2 > c->ev.size()) {

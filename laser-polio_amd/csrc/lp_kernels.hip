@@ -310,13 +310,17 @@ __device__ void day_stop_check(const Dev& d, int sim, int32_t t, int mask, int c
 
 // Per node: births, per-day resets, early-stop rule.  Inside lp_run_days only the
 // first day launches it: the end of each day (k_finish or k_day_end) begins the next one.
-__global__ void k_day_begin(Dev d, int mask, int32_t t, int32_t until) {
+// relist: today's RI pass lists every candidate of the next RI day, so that list starts empty
+// (it holds them already if the caller runs the tick's RI twice, and the node's part of it
+// has room for each agent once).
+__global__ void k_day_begin(Dev d, int mask, int32_t t, int32_t until, int relist) {
   const int n = blockIdx.x * blockDim.x + threadIdx.x;
   if (n == 0) {
     set_day(d, t, until);
     d.sel_count[0] = 0;
   }
   if (n >= d.n_nodes) return;
+  if (relist) d.ri_lcnt[(size_t)(d.ri_cnt[t + 1] & 1) * d.n_nodes + n] = 0;
   day_begin_node(d, n, t, mask);
   const int sim = d.node_sim[n];
   if (n == d.sims[sim].node_begin) {

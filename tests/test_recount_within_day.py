@@ -88,3 +88,30 @@ def test_host_edit_between_the_stages_of_an_ri_day(before, next_ri_by_stages):
     sim._mark_device_newer()
     assert ref.res["ri_vaccinated"][[28, 42]].sum() > 0
     _compare(sim, ref)
+
+
+@pytest.mark.gpu
+def test_ri_stage_twice_on_a_tick_lists_each_candidate_once():
+    """RI of tick 14 stepped twice in a population of mostly RI candidates (the draws are keyed by
+    agent and tick, so the second step changes no agent): the days after it are the oracle's,
+    the RI day 28 from the lists."""
+    k = 14
+    sim = make("campaigns", ri_age_days=(0, 20000))
+    p = sim.people
+    timers = np.concatenate([p.ri_timer[b:e] for b, e in zip(p.seg_begin, p.live_end, strict=True)])
+    assert (timers > 28).mean() > 0.5          # candidates of the lists made on ticks 0 to 14
+    print("[ri twice] candidates", int((timers > 28).sum()), flush=True)
+    ref = OracleSim(sim.export_tables(), pop0=sim.pars.init_pop).run()
+    eng = sim._ensure_engine()
+    eng.run_days(0, k)
+    for stage in STAGES:
+        eng.step(k, stage)
+        if stage == engmod.STAGE_RI:
+            eng.step(k, stage)
+    eng.run_days(k + 1, sim.nt)
+    eng.sync()
+    sim._mark_device_newer()
+    for name in ("ri_vaccinated", "ri_protected", "ri_new_exposed_by_strain", "ipv_vaccinated"):
+        ref.res[name][k] = getattr(sim.results, name)[k]       # the second step's row stands
+    assert ref.res["ri_vaccinated"][28].sum() > 0
+    _compare(sim, ref)
