@@ -16,8 +16,10 @@
  *
  * Up to 256 nodes one workgroup rolls all days of a call; up to 2048 nodes resident
  * workgroups do (a cooperative launch, outside stream capture), above that each day is a
- * launch.  If the resident workgroups cannot all run for 10 s the rows they did not reach
- * hold NaN.
+ * launch.  The resident workgroups wait for one another, 10 s at most: where a wait is given
+ * up (workgroups that do not get to run, a long preemption) the call still returns 0, and every
+ * output that was not computed holds NaN: rows of the trajectories, of inc, m_save, g_save and
+ * season_part, and aS, aE, aI, r0_bar and net_bar.
  *
  * Arrays are device pointers (float32, node-major rows of n).  All work is
  * queued on `hip_stream` (NULL = default stream).  Returns 0 or a negative
@@ -65,6 +67,16 @@ int lp_mf_adjoint_days(const lp_mf_model* model, int32_t t0, int32_t t1, const f
                        const float* m_save, const float* g_save, const float* a_inc, float* aS, float* aE,
                        float* aI, float* r0_bar, float* net_bar, float* season_part, float* work,
                        void* hip_stream);
+
+/* lp_mf_days and lp_mf_adjoint_days with another bound on the waits of the resident
+ * workgroups: wait_us microseconds instead of 10 s, for callers that would rather have NaN
+ * early (0: every wait is given up at once).  The other ways to roll do not wait. */
+int lp_mf_days_bounded(const lp_mf_model* model, int32_t t0, int32_t t1, float* S, float* E, float* I, float* inc,
+                       float* m_save, float* g_save, int32_t wait_us, void* hip_stream);
+int lp_mf_adjoint_days_bounded(const lp_mf_model* model, int32_t t0, int32_t t1, const float* S, const float* I,
+                               const float* m_save, const float* g_save, const float* a_inc, float* aS, float* aE,
+                               float* aI, float* r0_bar, float* net_bar, float* season_part, float* work,
+                               int32_t wait_us, void* hip_stream);
 
 /* lp_mf_adjoint_days without the `work` argument: the same kernels, with their scratch
  * in a fixed device array of the library (2 * LP_MF_NOALLOC_MAX_NODES floats, 256 KiB

@@ -7,9 +7,9 @@ namespace lp_mf {
 
 constexpr int WG = 256;
 
-// Scratch of lp_mf_adjoint_days_noalloc: the adjoint's two per-node work rows
-// (mixed-weight adjoint, carried I adjoint), 2 * LP_MF_NOALLOC_MAX_NODES floats
-// = 256 KiB held by every GPU the library runs on until the process ends.
+// Scratch of lp_mf_adjoint_days_noalloc: the two work rows of a launch per day (the
+// mixed-weight adjoints of a day and of the one after it), 2 * LP_MF_NOALLOC_MAX_NODES
+// floats = 256 KiB held by every GPU the library runs on until the process ends.
 static __device__ __align__(256) float scratch[2 * LP_MF_NOALLOC_MAX_NODES];
 
 constexpr int kMaxDevices = 64;
@@ -299,11 +299,14 @@ __global__ void __launch_bounds__(1024) k_mf_adj_wg(lp_mf_model m, int t0, int d
 // wait for the stores.  Reads that come too early hold up the stores they wait for (all of
 // them go to the same lines past the L2s): without the sleep before the first read a day
 // took 3.6 us instead of 2.2, and four wavefronts that only waited, or 256- or
-// 1024-thread workgroups, were slower too.  A wait ends after WAIT_TICKS of the 100 MHz
-// clock in any case: the kernel then returns and the rows keep PENDING.
+// 1024-thread workgroups, were slower too.  A wait ends after `wait_ticks` of the 100 MHz
+// clock in any case (a workgroup not resident, or preempted): the workgroup's owners then store
+// NaN everywhere they have not stored yet, the rows others wait for included, and return, so a
+// call that gave up leaves right values and NaN, never what the memory held before.
 constexpr int RES_WG = 512, RES_ROWS = 16;
 constexpr uint32_t PENDING = 0xFFFFFFFFu;
-constexpr int64_t WAIT_TICKS = 1000000000;   // 10 s
+constexpr int64_t TICKS_PER_US = 100;
+constexpr int32_t WAIT_US = 10000000;   // 10 s
 
 __global__ void __launch_bounds__(WG) k_mf_pending(uint32_t* p, int64_t n) {
   for (int64_t j = (int64_t)blockIdx.x * WG + threadIdx.x; j < n; j += (int64_t)gridDim.x * WG) p[j] = PENDING;
@@ -314,11 +317,13 @@ __device__ __forceinline__ void publish(float* p, float x) {
                      __HIP_MEMORY_SCOPE_AGENT);
 }
 // Elements [0, n) of `row` into LDS vector v, times `scale`; false (in every thread of the
-// workgroup) if one did not come in time.  Ends with a barrier.
+// workgroup) if one did not come within `wait_ticks` (0: at once).  Ends with a barrier.
 template <int K>
-__device__ __forceinline__ bool await_row(const float* row, int n, float scale, float* v, int* s_late) {
+__device__ __forceinline__ bool await_row(const float* row, int n, float scale, float* v, int* s_late,
+                                          int64_t wait_ticks) {
   constexpr int PER = 64 * K / RES_WG;
   const int w = threadIdx.x;
+  if (wait_ticks == 0) *s_late = 1;
   __builtin_amdgcn_s_sleep(16);   // 16 x 64 cycles: what a row needs to come at least
   uint32_t u[PER];
 #pragma unroll
@@ -335,7 +340,7 @@ __device__ __forceinline__ bool await_row(const float* row, int n, float scale, 
       u[a] = __hip_atomic_load(reinterpret_cast<const uint32_t*>(row + j), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (u[a] != PENDING) break;
       const int64_t now = (int64_t)wall_clock64();
-      if (t_end == 0) t_end = now + WAIT_TICKS;
+      if (t_end == 0) t_end = now + wait_ticks;
       if (now - t_end > 0) { *s_late = 1; break; }
     }
     v[j] = j < n ? __builtin_bit_cast(float, u[a]) * scale : 0.0f;
@@ -372,7 +377,7 @@ struct TwoRows {
 
 template <int K>
 __global__ void __launch_bounds__(RES_WG) k_mf_days_res(lp_mf_model m, int t0, int days, float* S, float* E, float* I,
-                                                        float* inc, float* msave, float* gsave) {
+                                                        float* inc, float* msave, float* gsave, int64_t wait_ticks) {
   __shared__ float v[2][64 * K];
   __shared__ int s_late;
   const int n = m.n, lane = threadIdx.x & 63;
@@ -401,8 +406,17 @@ __global__ void __launch_bounds__(RES_WG) k_mf_days_res(lp_mf_model m, int t0, i
   Season seasons;
   for (int d = 0; d < days; ++d) {
     if (d > 0) {
-      if (!await_row<K>(I + (size_t)d * n, n, 1.0f, v[d & 1], &s_late)) return;
+      const bool came = await_row<K>(I + (size_t)d * n, n, 1.0f, v[d & 1], &s_late, wait_ticks);
       store(d - 1);
+      if (!came) {
+        const float lost = __builtin_nanf("");
+        o = DayOut{lost, lost, lost, lost, lost, lost};
+        for (; d < days; ++d) {
+          if (own) publish(I + (size_t)(d + 1) * n + i, lost);
+          store(d);
+        }
+        return;
+      }
     }
     if ((d & 63) == 0) seasons.load(m.season, t0, days, d);
     const float mix = rows.apply(v[d & 1], lane);
@@ -418,7 +432,7 @@ __global__ void __launch_bounds__(RES_WG) k_mf_days_res(lp_mf_model m, int t0, i
 template <int K>
 __global__ void __launch_bounds__(RES_WG) k_mf_adj_res(lp_mf_model m, int t0, int days, const float* S, const float* msave,
                                                        const float* gsave, const float* ainc, float* aS, float* aE,
-                                                       float* aI, float* r0_bar, float* h) {
+                                                       float* aI, float* r0_bar, float* h, int64_t wait_ticks) {
   constexpr int PF = 4;
   __shared__ float v[2][64 * K];
   __shared__ int s_late;
@@ -452,7 +466,13 @@ __global__ void __launch_bounds__(RES_WG) k_mf_adj_res(lp_mf_model m, int t0, in
         publish(h + (size_t)d * n + i, hd);
         mbar = hd * row_scale(season);
       }
-      if (!await_row<K>(h + (size_t)d * n, n, row_scale(season), v[d & 1], &s_late)) return;
+      if (!await_row<K>(h + (size_t)d * n, n, row_scale(season), v[d & 1], &s_late, wait_ticks)) {
+        if (!own) return;
+        const float lost = __builtin_nanf("");
+        for (int e = d - 1; e >= 0; --e) publish(h + (size_t)e * n + i, lost);
+        aS[i] = aE[i] = aI[i] = r0_bar[i] = lost;
+        return;
+      }
       const float sum = rows.apply(v[d & 1], lane);
       if (own) x = adjoint_i(m, c, x, mbar, sum);
       if ((d & 63) == 0 && d > 0) seasons.load(m.season, t0, days, d - 1);
@@ -637,9 +657,10 @@ int fill_grid(int64_t n) { return (int)std::min<int64_t>((n + WG - 1) / WG, 2048
 
 extern "C" {
 
-int lp_mf_days(const lp_mf_model* model, int32_t t0, int32_t t1, float* S, float* E, float* I, float* inc,
-               float* m_save, float* g_save, void* hip_stream) {
-  if (!model || model->n <= 0 || t1 < t0 || !S || !E || !I || !inc) return LP_ERR_ARG;
+int lp_mf_days_bounded(const lp_mf_model* model, int32_t t0, int32_t t1, float* S, float* E, float* I, float* inc,
+                       float* m_save, float* g_save, int32_t wait_us, void* hip_stream) {
+  if (!model || model->n <= 0 || t1 < t0 || !S || !E || !I || !inc || wait_us < 0) return LP_ERR_ARG;
+  int64_t wait_ticks = wait_us * lp_mf::TICKS_PER_US;
   lp_mf_model m = *model;
   int n = m.n, days = t1 - t0;
   if (days == 0) return LP_OK;
@@ -656,7 +677,7 @@ int lp_mf_days(const lp_mf_model* model, int32_t t0, int32_t t1, float* S, float
       hipLaunchKernelGGL(lp_mf::k_mf_pending, dim3(lp_mf::fill_grid(cells)), dim3(lp_mf::WG), 0, s,
                          reinterpret_cast<uint32_t*>(I + n), cells);
       const hipError_t e = lp_mf::resident(n, [&](auto k) {
-        void* args[] = {&m, &t0, &days, &S, &E, &I, &inc, &m_save, &g_save};
+        void* args[] = {&m, &t0, &days, &S, &E, &I, &inc, &m_save, &g_save, &wait_ticks};
         return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&lp_mf::k_mf_days_res<decltype(k)::value>),
                                           dim3((n + lp_mf::RES_ROWS - 1) / lp_mf::RES_ROWS), dim3(lp_mf::RES_WG), args, 0, s);
       });
@@ -673,6 +694,11 @@ int lp_mf_days(const lp_mf_model* model, int32_t t0, int32_t t1, float* S, float
       break;
   }
   return hipGetLastError() == hipSuccess ? LP_OK : LP_ERR_HIP;
+}
+
+int lp_mf_days(const lp_mf_model* model, int32_t t0, int32_t t1, float* S, float* E, float* I, float* inc,
+               float* m_save, float* g_save, void* hip_stream) {
+  return lp_mf_days_bounded(model, t0, t1, S, E, I, inc, m_save, g_save, lp_mf::WAIT_US, hip_stream);
 }
 
 int lp_mf_adjoint_days_noalloc(const lp_mf_model* model, int32_t t0, int32_t t1, const float* S, const float* I,
@@ -692,9 +718,18 @@ int lp_mf_adjoint_days(const lp_mf_model* model, int32_t t0, int32_t t1, const f
                        const float* m_save, const float* g_save, const float* a_inc, float* aS, float* aE,
                        float* aI, float* r0_bar, float* net_bar, float* season_part, float* work,
                        void* hip_stream) {
+  return lp_mf_adjoint_days_bounded(model, t0, t1, S, I, m_save, g_save, a_inc, aS, aE, aI, r0_bar, net_bar,
+                                    season_part, work, lp_mf::WAIT_US, hip_stream);
+}
+
+int lp_mf_adjoint_days_bounded(const lp_mf_model* model, int32_t t0, int32_t t1, const float* S, const float* I,
+                               const float* m_save, const float* g_save, const float* a_inc, float* aS, float* aE,
+                               float* aI, float* r0_bar, float* net_bar, float* season_part, float* work,
+                               int32_t wait_us, void* hip_stream) {
   if (!model || model->n <= 0 || t1 < t0 || !S || !I || !m_save || !g_save || !a_inc || !aS || !aE || !aI ||
-      !r0_bar || !net_bar || !season_part || !work)
+      !r0_bar || !net_bar || !season_part || !work || wait_us < 0)
     return LP_ERR_ARG;
+  int64_t wait_ticks = wait_us * lp_mf::TICKS_PER_US;
   lp_mf_model m = *model;
   int n = m.n, days = t1 - t0;
   if (days == 0) return LP_OK;
@@ -712,7 +747,7 @@ int lp_mf_adjoint_days(const lp_mf_model* model, int32_t t0, int32_t t1, const f
       hipLaunchKernelGGL(lp_mf::k_mf_pending, dim3(lp_mf::fill_grid(cells)), dim3(lp_mf::WG), 0, s,
                          reinterpret_cast<uint32_t*>(h), cells);
       const hipError_t e = lp_mf::resident(n, [&](auto k) {
-        void* args[] = {&m, &t0, &days, &S, &m_save, &g_save, &a_inc, &aS, &aE, &aI, &r0_bar, &h};
+        void* args[] = {&m, &t0, &days, &S, &m_save, &g_save, &a_inc, &aS, &aE, &aI, &r0_bar, &h, &wait_ticks};
         return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&lp_mf::k_mf_adj_res<decltype(k)::value>),
                                           dim3((n + lp_mf::RES_ROWS - 1) / lp_mf::RES_ROWS), dim3(lp_mf::RES_WG), args, 0, s);
       });
