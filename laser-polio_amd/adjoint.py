@@ -11,9 +11,9 @@ Node compartments are aggregated from an ABM population at day 0 and rolled
 forward deterministically (expected exposures, daily E -> I and I -> R exits at
 the mean durations).  ``MeanFieldRollout`` is a torch.autograd.Function whose
 forward and hand-written adjoint run in liblpstep.so (lp_meanfield.h); a rollout
-too large to keep whole (KEEP_BYTES) keeps the state only every ``checkpoint``
-days and recomputes each segment forward before its adjoint.  ``rollout_reference`` is the same rollout in plain PyTorch
-ops, for autograd and finite-difference checks.
+too large to keep whole (``keep_bytes``) keeps the state only every ``checkpoint``
+days and recomputes each segment forward before its adjoint.  ``rollout_reference``
+is the same rollout in plain PyTorch ops, for autograd and finite-difference checks.
 """
 
 import ctypes
@@ -43,7 +43,8 @@ class LPMFModel(ctypes.Structure):
 
 
 # a rollout whose S, I, m and g trajectories (16 bytes a node and day) take no more than
-# this keeps them for its adjoint; a larger one is checkpointed and recomputed
+# this keeps them for its adjoint; a larger one is checkpointed and recomputed (the default of
+# rollout's keep_bytes)
 KEEP_BYTES = 256 << 20
 
 _mf = None
@@ -73,7 +74,8 @@ class MeanFieldRollout(torch.autograd.Function):
     """inc[t, i] = expected new exposures of node i on day t, t < len(season)."""
 
     @staticmethod
-    def forward(ctx, r0s, net, season, S0, E0, I0, rho, inv_pop, iota, inv_tau_e, inv_tau_i, checkpoint=30):
+    def forward(ctx, r0s, net, season, S0, E0, I0, rho, inv_pop, iota, inv_tau_e, inv_tau_i, checkpoint=30,
+                keep_bytes=None):
         dev = r0s.device
         if dev.type != "cuda":
             raise engmod.EngineUnavailable("the mean-field rollout runs on the HIP path (GPU tensors)")
@@ -93,7 +95,7 @@ class MeanFieldRollout(torch.autograd.Function):
         # a rollout whose trajectories are small is kept whole for the adjoint: one call over
         # all its days, nothing recomputed
         grad = any(ctx.needs_input_grad)
-        keep_all = checkpoint > 0 and 0 < 16 * T * n <= KEEP_BYTES
+        keep_all = checkpoint > 0 and 0 < 16 * T * n <= (KEEP_BYTES if keep_bytes is None else keep_bytes)
         state = [x.detach().to(**f32).reshape(1, n) for x in (S0, E0, I0)]
         checkpoints = []
         for t0 in range(0, T, T if keep_all else checkpoint):
@@ -143,11 +145,17 @@ class MeanFieldRollout(torch.autograd.Function):
                                              _p(net_bar), _p(season_part[t0:t1]), _p(work), stream),
                    "lp_mf_adjoint_days")
         season_bar = season_part.sum(dim=1)
-        return r0_bar, net_bar, season_bar, aS, aE, aI, None, None, None, None, None, None
+        return r0_bar, net_bar, season_bar, aS, aE, aI, None, None, None, None, None, None, None
 
 
-def rollout(r0s, net, season, S0, E0, I0, rho, inv_pop, iota, inv_tau_e, inv_tau_i, checkpoint=30):
-    return MeanFieldRollout.apply(r0s, net, season, S0, E0, I0, rho, inv_pop, iota, inv_tau_e, inv_tau_i, checkpoint)
+def rollout(r0s, net, season, S0, E0, I0, rho, inv_pop, iota, inv_tau_e, inv_tau_i, checkpoint=30, keep_bytes=None):
+    """inc[t, i] of MeanFieldRollout.  A rollout of up to ``keep_bytes`` (None: KEEP_BYTES) of
+    trajectories, 16 bytes a node and day, holds them until its backward; a larger one holds
+    the state of every ``checkpoint``-th day, 12 bytes a node, and needs one segment's
+    trajectories at a time.  ``keep_bytes=0`` always checkpoints, for programs that hold many
+    rollouts at once.  The results are the same bits either way."""
+    return MeanFieldRollout.apply(r0s, net, season, S0, E0, I0, rho, inv_pop, iota, inv_tau_e, inv_tau_i, checkpoint,
+                                  keep_bytes)
 
 
 def rollout_reference(r0s, net, season, S0, E0, I0, rho, inv_pop, iota, inv_tau_e, inv_tau_i):
