@@ -464,10 +464,12 @@ __device__ __forceinline__ EIConst ei_const(const lp_sim_params& sp) {
 
 // ri_timer <- actual values: for live agents that are not chronically missed,
 // minus RI's decrements from the reference tick through the latest applied RI
-// step (one workgroup per span); k_set_ri_ref then moves the reference there.
+// step (one workgroup per span); k_set_ri_ref then moves the reference there.  A
+// simulation that stopped had its last RI step on or before its stop day.
 __global__ void __launch_bounds__(WG) k_ri_sync(Dev d) {
   const int4 span = d.spans[blockIdx.x];
-  const int32_t dc = d.ri_cnt[d.ri_ref[1] + 1] - d.ri_cnt[d.ri_ref[0] + 1];
+  const int32_t stop = d.stop_day[span.w], r0 = d.ri_ref[0], r1 = d.ri_ref[1];
+  const int32_t dc = d.ri_cnt[(r1 < stop ? r1 : stop) + 1] - d.ri_cnt[(r0 < stop ? r0 : stop) + 1];
   const int32_t shift = d.sims[span.w].ri_step * dc;
   if (shift == 0) return;
   for (int u = 0; u < span.z; ++u) {
@@ -1314,8 +1316,9 @@ __global__ void __launch_bounds__(WG) k_ri_list(Dev d, int mask) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int sim = d.node_sim[n];
   const int32_t flags = stage_day_flags(dy.y, mask);
-  if (sim_stopped(d, sim, t) || !(flags & LP_DAY_RI)) return;
-  if (n == 0 && blockIdx.y == 0 && tid == 0) d.ri_ref[1] = t;
+  if (!(flags & LP_DAY_RI)) return;
+  if (n == 0 && blockIdx.y == 0 && tid == 0) d.ri_ref[1] = t;   // (node 0's simulation may have stopped)
+  if (sim_stopped(d, sim, t)) return;
   const lp_sim_params& sp = d.sims[sim];
   const int32_t step = sp.ri_step;
   const int32_t sh_today = step * (dy.w - d.ri_cnt[d.ri_ref[0] + 1]);
@@ -1467,6 +1470,7 @@ __global__ void __launch_bounds__(WG, 5) k_full(Dev d, int mask) {
   const int64_t live_hi = d.live_end[node];
   const int32_t stop_day = d.stop_day[sim];
   const int32_t flags = stage_day_flags(dy.y, mask);
+  if (RI && (flags & LP_DAY_RI) && blockIdx.x == 0 && tid == 0) d.ri_ref[1] = t;
   if (stop_day < t) return;
   const int want = ((flags & LP_DAY_VD_STEP) ? FULL_VD : 0) | ((flags & LP_DAY_RI) ? FULL_RI : 0) |
                    ((flags & LP_DAY_SIA) ? FULL_SIA : 0);
@@ -1510,7 +1514,6 @@ __global__ void __launch_bounds__(WG, 5) k_full(Dev d, int mask) {
   const int32_t cnt_ref = d.ri_cnt[d.ri_ref[0] + 1];
   const int32_t sh_prev = sp.ri_step * (dy.z - cnt_ref);
   const int32_t sh_today = sp.ri_step * (dy.w - cnt_ref);
-  if (RI && blockIdx.x == 0 && tid == 0) d.ri_ref[1] = t;
   // does any of today's campaigns target this node?  (uniform over the workgroup)
   bool sia_here = false;
   if (SIA)
