@@ -907,7 +907,7 @@ def adjoint_workload(args):
     ABM run on the GPU at the known parameters; gradient at perturbed parameters (r0_scalars
     x 0.9, gravity k x 0.8, amplitude x 1.2) with respect to the 774 r0_scalars, gravity
     k, a, b, c and seasonal amplitude and peak.  Reported: seconds per loss + gradient
-    (HIP forward and adjoint, 30-day checkpoints), relative error against autograd of the
+    (HIP forward and adjoint, trajectories kept), relative error against autograd of the
     plain float32 PyTorch rollout (per parameter group) and against float64 central
     differences (h = 1e-4 relative) on scalars and a sample of r0_scalars."""
     scale = 0.1 if args.scale == 1.0 else args.scale
@@ -980,7 +980,7 @@ def adjoint_result(scale, init="device"):
     log(f"[bench] loss {L_hip:.6e}; HIP forward+adjoint {ms:.2f} ms (autograd of plain float32 rollout {t_ag * 1e3:.1f} ms)")
     log(f"[bench] relative error vs autograd: {max(rel_ag.values()):.2e}; vs central differences: {max(fd_err.values()):.2e}")
     out = {
-        "metric": "mean-field adjoint: loss + gradient time (774 nodes, 180 days, 30-day checkpoints)",
+        "metric": "mean-field adjoint: loss + gradient time (774 nodes, 180 days)",
         "value": round(ms, 3),
         "unit": "ms",
         "n_gpus": 1,

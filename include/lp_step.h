@@ -161,8 +161,9 @@ int lp_log(lp_ctx* ctx, int32_t t);
 
 /* The caller changed bound buffers between steps (the reference lets host code
  * edit sim.people / sim.results between component steps, e.g. seed_schedule
- * injections, model.py:772-786).  The next agent pass recounts the per-node and
- * per-chunk susceptible statistics the library otherwise carries from day to day. */
+ * injections, model.py:772-786).  The next call recounts everything the library otherwise
+ * carries from day to day (per-node counts, per-chunk susceptible weights, lists), between
+ * two days or between two stage calls of one. */
 int lp_invalidate(lp_ctx* ctx);
 
 /* Population initialisation on the device, in place of the host draws of the
@@ -224,7 +225,9 @@ typedef struct {
  * context) and the distances (device, float64, each simulation's n x n block row-major at
  * the same offset as its "network_t" block).  Replaces the host construction of
  * model.py:1213-1258 for calibration loops that rebuild networks per trial.  Takes effect
- * from the next simulated day; queued on the context stream. */
+ * from the next simulated day; queued on the context stream.  The first call allocates
+ * device scratch that the context keeps: 8 bytes per network entry (less time per build;
+ * without room for it the build does without), 24 per node, one spec per simulation. */
 int lp_build_network(lp_ctx* ctx, const lp_gravity_spec* specs, int32_t n_sims, const double* pop,
                      const double* dist);
 

@@ -189,7 +189,7 @@ constexpr int kSampleGrid = 2048;
 constexpr int kRiSplit = 8;
 
 
-// Host-side mirror of the device day classification (k_agents::is_plain_day).
+// Host-side mirror of the device day classification (lp::stage_day_flags).
 int32_t host_stage_flags(int32_t flags, int mask) {
   int32_t f = 0;
   if (mask & LP_STAGE_VITAL) f |= flags & (LP_DAY_VD_STEP | LP_DAY_VD_COPY);

@@ -21,7 +21,9 @@ __device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
 // as 1, 2, 3", SC'11): 10 rounds of two 32x32->64 multiplies with Weyl key bumps.  Each
 // product is one 64-bit multiply-add and each output word one three-input xor (written as
 // high and low halves, twice the quarter-rate multiplies: the draws of 269 M agents took
-// 7.5 ms instead of 5.4).
+// 7.5 ms instead of 5.4).  The 64-bit products come in register pairs, which costs the kernels
+// that draw in the middle of other work 10 to 20 registers (k_ei, k_vd, and k_full, which now
+// spills a few at the times it had).
 __device__ __forceinline__ uint4 philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint64_t seed) {
   uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
 #pragma unroll

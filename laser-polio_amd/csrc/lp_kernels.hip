@@ -366,7 +366,7 @@ __device__ __forceinline__ void static_for(F&& f) {
 //            state column and the E/I columns of quads holding an E or I agent
 //   FULL     VD step / RI / SIA days: births, deaths and the campaigns too
 // FULL days use kinds 1..7 (FULL_* bits); KIND_PLAIN_LIST: a plain day from the E / I list (k_ei);
-// KIND_FULL_LIST + F - 1: FULL day F with DiseaseState from the list (k_ei, then k_full<F, false>)
+// KIND_FULL_LIST + F - 1: FULL day F with DiseaseState from the list (k_ei, then k_vd, k_ri_list, k_sia)
 enum : int { KIND_PLAIN = 0, KIND_FULL = 1, KIND_PLAIN_LIST = 8, KIND_FULL_LIST = 9, N_KINDS = 16 };
 
 __device__ __forceinline__ bool is_plain_day(int32_t flags) {
@@ -597,8 +597,8 @@ __device__ __forceinline__ uint4* ei_list_of(const Dev& d, int b, int node) {
   return d.ei_list + (size_t)b * (size_t)d.capacity + d.seg_begin[node];
 }
 
-// Appends one entry (one atomic, returning); for the rare path (inline DiseaseState)
-// that appends from divergent code.
+// Appends one entry (one atomic, returning); for the rare paths that append from divergent
+// code: inline DiseaseState and round-1 winners of a node without reserved positions.
 __device__ __forceinline__ void append_entry(const Dev& d, int b, int node, const uint4& e) {
   const int pos = atomicAdd(d.ei_cnt + (size_t)b * d.n_nodes + node, 1);
   ei_list_of(d, b, node)[pos] = e;
@@ -1057,7 +1057,8 @@ __global__ void __launch_bounds__(WG) k_plain(Dev d, int mask) {
 // the place in tomorrow's list (8 us).  So a piece's reads of one kind go out together:
 // the transitions of its four entries per lane first (entries alone), then the records of
 // its paralysis rolls beside the atomic for its survivors' places (one entry after the
-// other: 64 replicates at their peak 91 -> 83 us, the year 70.8 -> 69.9 ms).
+// other: 64 replicates at their peak 91 -> 83 us, the year 70.8 -> 69.9 ms).  The four entries
+// of a lane live through both: 85 VGPRs, 5 waves per SIMD.
 
 // Exclusive prefix over n in [0, N) of cnt(n), by every thread of one workgroup:
 // emit(n, prefix) for each n; returns the total.  Each pass takes 4 * WG nodes, 4
@@ -1449,7 +1450,9 @@ __global__ void __launch_bounds__(WG) k_ri_list(Dev d, int mask) {
 // births and deaths are compacted per wave for disease progression and the
 // E / I tally, as on plain days.  Agents exposed by RI or SIA today are
 // tallied as E directly and are not progressed (DiseaseState runs before RI and
-// SIA in the reference day, model.py:226-241).
+// SIA in the reference day, model.py:226-241).  Held to 5 waves per SIMD, 20 to 40 bytes a
+// lane spill; each kind takes what it took without them (4.6 M agents of 14 nodes, births and
+// deaths 290 us, RI 540, SIA 590, all three 880, means over five heavy days).
 enum : int { FULL_VD = 1, FULL_RI = 2, FULL_SIA = 4 };
 
 template <int F, bool EI>
@@ -3018,11 +3021,6 @@ __device__ __forceinline__ bool claim_from(int8_t* state, int64_t slot, uint32_t
   }
 }
 
-// Remove an exposed agent's weight from its chunk and its span.
-__device__ __forceinline__ void unweight(const Dev& d, int node, int64_t slot) {
-  unweight_in(d, span_of(d, node, slot), slot, weight_q24(d.risk[slot]));
-}
-
 // The strain of a selected agent, drawn by cumulative strain probability
 // (model.py:1125-1147) against the node's thresholds thr[0..K) (already loaded).
 __device__ __forceinline__ int strain_draw(const Dev& d, const uint64_t* thr, uint64_t seed, int64_t slot_base,
@@ -3533,7 +3531,9 @@ __device__ __forceinline__ void finish_node(const Dev& d, int32_t t, int n, int3
 // year with it / with its work by one thread at the end of k_finish / as here: 774 nodes
 // 33.5 / 32.2 / 31.4 ms, 14 nodes 22.9 / 22.0 / 21.4 ms, 64 replicates 69.7 / 67.8 / 67.2 ms,
 // 5000 nodes x 150 days 27.5 / 27.5 / 27.1 ms.  (One thread that loads from the start holds
-// forty registers and as many pointers, which the sampling rounds then spill.)
+// forty registers and as many pointers: 200 bytes of scratch a lane in k_finish<512, 6>.
+// One register and the addresses still cost it some: 48 bytes, of which the rounds alone
+// take 36.)
 enum : int { CL_S, CL_R, CL_POTP, CL_P, CL_NEWEXP, CL_RR, CL_POP, CL_E, CL_I = CL_E + LP_MAX_STRAINS,
              CL_BS = CL_I + LP_MAX_STRAINS, CL_CS = CL_BS + LP_MAX_STRAINS, CL_CSPOS = CL_CS + 2,
              CL_RATE = CL_CSPOS + 2, CL_LIVE = CL_RATE + 2, CL_SEG = CL_LIVE + 2, CL_SEED = CL_SEG + 2,

@@ -622,6 +622,11 @@ __global__ void __launch_bounds__(WG) k_mf_season(lp_mf_model m, int t0, int day
 
 // Which way a call goes.  The one-workgroup kernels lead the resident ones up to the 256
 // nodes whose rows their registers hold; above 2048 nodes two rows a wavefront no longer fit.
+// A cooperative launch costs about 20 us more than an ordinary one, so calls of few days
+// were faster a launch per day (774 nodes, forward 1 / 5 / 30 / 180 days: 36 / 43 / 89 / 360 us
+// against 16 / 32 / 165 / 850; adjoint 45 / 53 / 98 / 367 against 21 / 76 / 267 / 1555).
+// The choice goes by the nodes alone all the same: the ways add in different orders, and days
+// in one call or in several are to give the same bits.
 enum class Path { kOneWorkgroup, kResident, kPerDay };
 constexpr int ONE_WG_MAX = 256, RES_MAX = 2048;
 
