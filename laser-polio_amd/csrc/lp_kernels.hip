@@ -1045,7 +1045,7 @@ __global__ void __launch_bounds__(WG) k_plain(Dev d, int mask) {
 // DiseaseState and the E / I tally from the E / I list: the agents in list
 // t & 1 only (no other agent is E or I), survivors appended to list (t + 1) & 1.
 // On plain days this is the whole agent pass; on FULL days it runs first and
-// k_full<F, false> then does births, deaths, RI and SIA.  On VD step days the
+// k_vd, k_ri_list and k_sia then do births, deaths, RI and SIA.  On VD step days the
 // agents due to die today are skipped: the reference removes them before
 // DiseaseState (model.py:226-241), so neither step sees them.  Each wavefront takes
 // pieces of EI_PIECE entries of one node (ei_piece_off) in turn and adds the
