@@ -300,9 +300,10 @@ __global__ void __launch_bounds__(1024) k_mf_adj_wg(lp_mf_model m, int t0, int d
 // them go to the same lines past the L2s): without the sleep before the first read a day
 // took 3.6 us instead of 2.2, and four wavefronts that only waited, or 256- or
 // 1024-thread workgroups, were slower too.  A wait ends after `wait_ticks` of the 100 MHz
-// clock in any case (a workgroup not resident, or preempted): the workgroup's owners then store
-// NaN everywhere they have not stored yet, the rows others wait for included, and return, so a
-// call that gave up leaves right values and NaN, never what the memory held before.
+// clock in any case (a workgroup not resident, or preempted).  The workgroup's owners then store
+// NaN everywhere they have not stored yet and return; the rows that others wait for keep
+// PENDING, a NaN itself.  So a call that gave up leaves right values and NaN, never what the
+// memory held before.
 constexpr int RES_WG = 512, RES_ROWS = 16;
 constexpr uint32_t PENDING = 0xFFFFFFFFu;
 constexpr int64_t TICKS_PER_US = 100;
@@ -317,13 +318,12 @@ __device__ __forceinline__ void publish(float* p, float x) {
                      __HIP_MEMORY_SCOPE_AGENT);
 }
 // Elements [0, n) of `row` into LDS vector v, times `scale`; false (in every thread of the
-// workgroup) if one did not come within `wait_ticks` (0: at once).  Ends with a barrier.
+// workgroup) if one did not come within `wait_ticks`, or *s_late was set.  Ends with a barrier.
 template <int K>
 __device__ __forceinline__ bool await_row(const float* row, int n, float scale, float* v, int* s_late,
                                           int64_t wait_ticks) {
   constexpr int PER = 64 * K / RES_WG;
   const int w = threadIdx.x;
-  if (wait_ticks == 0) *s_late = 1;
   __builtin_amdgcn_s_sleep(16);   // 16 x 64 cycles: what a row needs to come at least
   uint32_t u[PER];
 #pragma unroll
@@ -382,7 +382,7 @@ __global__ void __launch_bounds__(RES_WG) k_mf_days_res(lp_mf_model m, int t0, i
   __shared__ int s_late;
   const int n = m.n, lane = threadIdx.x & 63;
   const int i0 = blockIdx.x * RES_ROWS + (threadIdx.x >> 6) * 2, i = i0 + lane;
-  if (threadIdx.x == 0) s_late = 0;
+  if (threadIdx.x == 0) s_late = wait_ticks == 0;
   for (int j = threadIdx.x; j < 64 * K; j += RES_WG) v[0][j] = j < n ? I[j] : 0.0f;
   __syncthreads();
   TwoRows<K> rows;
@@ -411,10 +411,7 @@ __global__ void __launch_bounds__(RES_WG) k_mf_days_res(lp_mf_model m, int t0, i
       if (!came) {
         const float lost = __builtin_nanf("");
         o = DayOut{lost, lost, lost, lost, lost, lost};
-        for (; d < days; ++d) {
-          if (own) publish(I + (size_t)(d + 1) * n + i, lost);
-          store(d);
-        }
+        for (; d < days; ++d) store(d);
         return;
       }
     }
@@ -438,7 +435,7 @@ __global__ void __launch_bounds__(RES_WG) k_mf_adj_res(lp_mf_model m, int t0, in
   __shared__ int s_late;
   const int n = m.n, lane = threadIdx.x & 63;
   const int i0 = blockIdx.x * RES_ROWS + (threadIdx.x >> 6) * 2, i = i0 + lane;
-  if (threadIdx.x == 0) s_late = 0;
+  if (threadIdx.x == 0) s_late = wait_ticks == 0;
   __syncthreads();
   Season seasons;
   seasons.load(m.season, t0, days, days - 1);
@@ -467,10 +464,7 @@ __global__ void __launch_bounds__(RES_WG) k_mf_adj_res(lp_mf_model m, int t0, in
         mbar = hd * row_scale(season);
       }
       if (!await_row<K>(h + (size_t)d * n, n, row_scale(season), v[d & 1], &s_late, wait_ticks)) {
-        if (!own) return;
-        const float lost = __builtin_nanf("");
-        for (int e = d - 1; e >= 0; --e) publish(h + (size_t)e * n + i, lost);
-        aS[i] = aE[i] = aI[i] = r0_bar[i] = lost;
+        if (own) aS[i] = aE[i] = aI[i] = r0_bar[i] = __builtin_nanf("");
         return;
       }
       const float sum = rows.apply(v[d & 1], lane);
@@ -623,7 +617,7 @@ __global__ void __launch_bounds__(WG) k_mf_season(lp_mf_model m, int t0, int day
 // Which way a call goes.  The one-workgroup kernels lead the resident ones up to the 256
 // nodes whose rows their registers hold; above 2048 nodes two rows a wavefront no longer fit.
 // A cooperative launch costs about 20 us more than an ordinary one, so calls of few days
-// were faster a launch per day (774 nodes, forward 1 / 5 / 30 / 180 days: 36 / 43 / 89 / 360 us
+// were faster a launch per day (774 nodes, forward 1 / 5 / 30 / 180 days: 36 / 43 / 84 / 340 us
 // against 16 / 32 / 165 / 850; adjoint 45 / 53 / 98 / 367 against 21 / 76 / 267 / 1555).
 // The choice goes by the nodes alone all the same: the ways add in different orders, and days
 // in one call or in several are to give the same bits.
